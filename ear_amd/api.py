@@ -64,7 +64,8 @@ class Context:
         lanes, 2 closest-hit lanes refilled from the queue, 3 both kernels
         refilled (default); refill / fetch_chunk: idle lanes that trigger a
         refill (default 24), entries claimed per atomic (default: one per
-        idle lane) and queue segments with a counter each (default 64);
+        idle lane; 64 while the queue is long) and queue segments with a
+        counter each (default 16);
         graph_iters > 0 replays the bounce loop as a captured HIP graph;
         tail_rays: the last <= tail_rays live rays go to one launch that
         traces each to its end (default: every ray when no scene of the call

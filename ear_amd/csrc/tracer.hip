@@ -93,6 +93,9 @@ struct Fetch {
 };
 constexpr uint32_t kSegStride = 32;  // uint32 words per counter line
 constexpr uint32_t kMaxSeg = 64;
+// a batch of 32 rooms: 174 ms at 16 segments, 177 at 64, 177 at 8; the
+// 200k-triangle hall: 375, 377, 374
+constexpr uint32_t kSegDefault = 16;
 
 // ---------------------------------------------------------------------------
 // wave helpers
@@ -257,46 +260,62 @@ __device__ __forceinline__ void stat_drops(unsigned long long* stats, const Drop
         atomicMax(stats + (size_t)(blockIdx.x % kStatCopies) * ST_N + ST_BINS, (unsigned long long)e);
 }
 
-// Lane refilling (see Fetch): call with the whole wave when !exhausted and at
-// least f.refill lanes are idle (or all are); `act` is the ballot of busy
-// lanes.  Returns the queue entry handed to this lane, or ~0u.  The queue
-// [0, n) is cut into f.n_seg segments with a counter each, so that claims of
-// many waves do not serialise on one address: a wave claims from its current
-// segment `seg` and moves on to the next one when that is used up; after
-// f.n_seg used-up segments in a row everything has been taken.
-__device__ __forceinline__ uint32_t take_entries(const Fetch& f, uint32_t n, uint64_t act, uint32_t lane,
-                                                 uint32_t& c_next, uint32_t& c_end, bool& exhausted,
-                                                 uint32_t& seg) {
-    const uint32_t n_idle = 64u - (uint32_t)__popcll(act);
-    if (c_next == c_end) {
-        // claim f.chunk entries, or exactly one per idle lane
-        const uint32_t want = f.chunk ? f.chunk : n_idle;
-        for (uint32_t fails = 0;;) {
-            const uint32_t lo = (uint32_t)(((uint64_t)n * seg) / f.n_seg);
-            const uint32_t hi = (uint32_t)(((uint64_t)n * (seg + 1)) / f.n_seg);
-            uint32_t old = 0;
-            if (lo < hi && lane == 0) old = atomicAdd(f.counter + seg * kSegStride, want);
-            old = __shfl(old, 0);
-            if (lo < hi && old < hi - lo) {
-                c_next = lo + old;
-                c_end = min(lo + old + want, hi);
-                break;
-            }
-            if (++fails == f.n_seg) {
-                exhausted = true;
-                c_next = c_end = 0;
-                break;
-            }
-            seg = seg + 1 == f.n_seg ? 0 : seg + 1;
+// Queue entries handed to the lanes of a wave (see Fetch).  The queue [0, n)
+// is cut into f.n_seg segments with a counter each, so that claims of many
+// waves do not serialise on one address: a wave claims from its current
+// segment and moves on to the next one when that is used up; after f.n_seg
+// used-up segments in a row everything has been taken.  A queue no longer
+// than the grid's lanes needs no claim: each wave has its own 64 entries (the
+// blocks' first waves before the second ones, so that a short queue spreads
+// over all CUs) and the waves past its end leave at once; trying the
+// segments in turn to learn that nothing is left took such launches longer
+// than their walks (400 bounces of 0.5M rays in a room, 64 segments: 22 ms,
+// 8 ms without).  The state is the same in the whole wave and kept in scalar
+// registers, and no claim divides (with a segment's bounds formed per lane
+// and claim in 64 bits a refill cost about 300 instructions).
+struct Claim {
+    uint32_t n, next, end, seg, seg_len, n_seg, want, fails;
+    __device__ __forceinline__ Claim(uint32_t n_, uint32_t gtid, uint32_t threads, const Fetch& f) {
+        n = (uint32_t)__builtin_amdgcn_readfirstlane((int)n_);
+        n_seg = f.n_seg;
+        seg = (uint32_t)__builtin_amdgcn_readfirstlane((int)((gtid >> 6) % n_seg));
+        seg_len = n / n_seg + (n % n_seg ? 1u : 0u);
+        next = end = fails = 0;
+        // entries per atomic: what one refill needs, or while the queue is
+        // long (256 for every wave) enough for several refills
+        want = f.chunk ? f.chunk : (n / 256u >= threads / 64u ? 64u : 0u);
+        if (n <= threads) {
+            const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)((threadIdx.x >> 6) * gridDim.x + blockIdx.x));
+            next = min(wave * 64u, n);
+            end = min(next + 64u, n);
+            fails = n_seg;
         }
     }
-    const uint64_t idle = ~act;
-    const uint32_t avail = c_end - c_next;
-    const uint32_t rank = (uint32_t)__popcll(idle & ((1ull << lane) - 1ull));
-    const uint32_t mine = c_next + rank;
-    c_next += min(avail, n_idle);
-    return (((act >> lane) & 1ull) == 0 && rank < avail) ? mine : 0xFFFFFFFFu;
-}
+    __device__ __forceinline__ bool exhausted() const { return fails >= n_seg && next >= end; }
+    // the whole wave; idle: the ballot of its idle lanes.  The entry handed to
+    // this lane, or ~0u.
+    __device__ __forceinline__ uint32_t take(const Fetch& f, uint64_t idle, uint32_t lane) {
+        const uint32_t n_idle = (uint32_t)__popcll(idle);
+        while (next >= end && fails < n_seg) {
+            const uint32_t lo = min(seg * seg_len, n), hi = min(lo + seg_len, n), k = want ? want : n_idle;
+            uint32_t old = 0;
+            if (lane == 0) old = atomicAdd(f.counter + seg * kSegStride, k);
+            old = (uint32_t)__builtin_amdgcn_readfirstlane((int)old);
+            if (old < hi - lo) {
+                next = lo + old;
+                end = min(next + k, hi);
+                fails = 0;
+            } else {
+                ++fails;
+                seg = seg + 1 == n_seg ? 0u : seg + 1;
+            }
+        }
+        const uint32_t rank = (uint32_t)__popcll(idle & ((1ull << lane) - 1ull));
+        const uint32_t avail = end - next, base = next;
+        next += min(avail, n_idle);
+        return (((idle >> lane) & 1ull) && rank < avail) ? base + rank : 0xFFFFFFFFu;
+    }
+};
 
 // ---------------------------------------------------------------------------
 // BVH traversal
@@ -340,34 +359,42 @@ __device__ __forceinline__ void slab(const SlabRay& r, float lx, float ly, float
 
 // Per-thread traversal stack: the first LDS entries in shared memory
 // (column-major over the block so a wave's accesses are conflict free), the
-// rest in a global overflow area indexed [entry][persistent thread].
+// rest in a global overflow area indexed [entry][persistent thread].  The
+// pointers carry their address space: a choice between two generic pointers
+// compiles to flat accesses, which go through the global memory's address
+// unit even when they hit LDS.
+typedef __attribute__((address_space(3))) int LdsInt;
+typedef __attribute__((address_space(1))) int GlobalInt;
 template <int LDS, int BLOCK>
 struct Stack {
-    int* lds;
-    int* gstack;
-    uint32_t gtid, gthreads;
+    LdsInt* lds;
+    GlobalInt* over;
+    uint32_t n_over;  // persistent threads sharing the overflow area
     int sp = 0;
-    __device__ __forceinline__ int* slot(int i) const {
-        return i < LDS ? lds + i * BLOCK : gstack + (size_t)(i - LDS) * gthreads + gtid;
-    }
+    __device__ __forceinline__ Stack(int* lds_, int* gstack, uint32_t gtid, uint32_t gthreads)
+        : lds((LdsInt*)lds_), over((GlobalInt*)gstack + gtid), n_over(gthreads) {}
     __device__ __forceinline__ void push(int v) {
-        *slot(sp) = v;
+        if (__builtin_expect(sp < LDS, 1))
+            lds[sp * BLOCK] = v;
+        else
+            over[(size_t)(uint32_t)(sp - LDS) * n_over] = v;
         ++sp;
     }
     __device__ __forceinline__ int pop() {
         --sp;
-        return *slot(sp);
+        if (__builtin_expect(sp < LDS, 1)) return lds[sp * BLOCK];
+        return over[(size_t)(uint32_t)(sp - LDS) * n_over];
     }
 };
 
 // Tests the triangles of leaf reference `cref`.  Closest hit (ANY = false):
 // t in (0.001, best_t) with the lower original index winning ties, as the
 // reference's strict '<' scan does (src/Mesh.cpp:39-45).  Any hit (ANY =
-// true): segment parameter t in (1e-5, 1) (src/Mesh.cpp:58-71); returns true
-// as soon as one is found.
+// true): segment parameter t in (1e-5, 1) (src/Mesh.cpp:58-71); best_s = 0 as
+// soon as one is found.
 template <bool ANY, bool INSTR>
-__device__ __forceinline__ bool test_leaf(const Traversal& T, int32_t cref, V3 o, V3 d, float& best_t, int& best_s,
-                                          uint32_t& best_o, bool& found, uint32_t& ntri) {
+__device__ __forceinline__ void test_leaf(const Traversal& T, int32_t cref, V3 o, V3 d, float& best_t, int& best_s,
+                                          uint32_t& best_o, uint32_t& ntri) {
     uint32_t u = (uint32_t)cref;
     uint32_t first = u & 0x00FFFFFFu;
     uint32_t cnt = ((u >> 24) & 0x7Fu) + 1;
@@ -378,165 +405,61 @@ __device__ __forceinline__ bool test_leaf(const Traversal& T, int32_t cref, V3 o
         if (INSTR) ++ntri;
         if (mt_intersect(v0, e1, e2, o, d, t)) {
             if (ANY) {
-                if (t > 1e-5f && t < 1.0f) return true;
+                if (t > 1e-5f && t < 1.0f) {
+                    best_s = 0;
+                    return;
+                }
             } else {
                 uint32_t orig = __float_as_uint(t2.y);
                 if (t > 0.001f && (t < best_t || (t == best_t && orig < best_o))) {
                     best_t = t;
                     best_s = (int)i;
                     best_o = orig;
-                    found = true;
                 }
             }
         }
     }
-    return false;
 }
 
-// a_k by masks (a chain of selects on k would be turned into an indexed
-// array in scratch memory)
-__device__ __forceinline__ uint32_t sel4(int k, uint32_t a0, uint32_t a1, uint32_t a2, uint32_t a3) {
-    return (a0 & (0u - (uint32_t)(k == 0))) | (a1 & (0u - (uint32_t)(k == 1))) | (a2 & (0u - (uint32_t)(k == 2))) |
-           (a3 & (0u - (uint32_t)(k == 3)));
-}
-
-__device__ __forceinline__ void cswap(float& ka, int& va, float& kb, int& vb) {
-    if (kb < ka) {
-        float tk = ka;
-        ka = kb;
-        kb = tk;
-        int tv = va;
-        va = vb;
-        vb = tv;
-    }
-}
-
-// One ray's BVH walk as a resumable state machine, so that a persistent lane
-// can interleave the walks of rays it fetches one after another.  4-wide
-// tree: a step either tests one pending leaf (nearest first; for the closest
-// hit a leaf whose box starts beyond the best hit so far is dropped) or
-// visits one internal node, whose hit children are sorted by entry distance:
-// leaves become pending (a bit mask over the sorted children), the nearest
-// internal child is visited next and the others are pushed.  One leaf per step keeps a wave's triangle tests in one
-// code path instead of one per child slot.  2-wide tree: a step visits one
-// node and tests its leaf children at once.  Closest hit (ANY = false):
-// best_* hold the nearest hit so far (order independent: ties go to the lower
-// original index).  Any hit: `found` is set when a blocker is found.
+// A walk of one ray as a resumable state machine, so that a persistent lane
+// can interleave the walks of rays it fetches one after another.  Closest hit
+// (ANY = false): best_* hold the nearest hit so far (order independent: ties
+// go to the lower original index).  Any hit: best_s = 0 once a blocker is
+// found.
+//   idle()   no walk (or it has ended)
+//   start()  begins one (an empty scene's ends at once)
+//   step()   one step of every lane's walk, called by all (active) lanes of
+//            the wave; true for a lane whose walk has just ended
+//
+// 2-wide tree: a step visits one node and tests its leaf children at once.
 template <int LDS, int BLOCK, int WIDTH, bool ANY, bool INSTR>
 struct Walker {
+    static constexpr int kIdle = kEmpty4;
     SlabRay sr;
     V3 o, d;
-    float best_t;
-    int best_s;
-    uint32_t best_o;
-    int node;  // next internal node to visit, -1: pop one
-    bool found;
-    uint32_t pend;             // 4-wide tree: bit k set = child k of the last node is a leaf to test
-    int pr0, pr1, pr2, pr3;    // that node's children, sorted by entry distance
-    float pk0, pk1, pk2, pk3;  // and their entry distances
+    float best_t = 0.0f;
+    int best_s = -1;
+    uint32_t best_o = 0;
+    int node = kIdle;  // next internal node to visit, -1: pop one
     Stack<LDS, BLOCK> stk;
 
     __device__ __forceinline__ Walker(int* lds, int* gstack, uint32_t gtid, uint32_t gthreads)
-        : stk{lds, gstack, gtid, gthreads} {}
-
-    // returns false when the walk is already over (empty scene)
-    __device__ __forceinline__ bool start(const Traversal& T, V3 o_, V3 d_, float t_max) {
+        : stk(lds, gstack, gtid, gthreads) {}
+    __device__ __forceinline__ bool idle() const { return node == kIdle; }
+    __device__ __forceinline__ bool found() const { return best_s >= 0; }
+    __device__ __forceinline__ void start(const Traversal& T, V3 o_, V3 d_, float t_max) {
         o = o_;
         d = d_;
         sr = SlabRay{o.x, o.y, o.z, safe_inv(d.x), safe_inv(d.y), safe_inv(d.z)};
         best_t = t_max;
         best_s = -1;
         best_o = 0;
-        node = 0;
-        found = false;
-        pend = 0;
+        node = T.n_tris != 0 ? 0 : kIdle;
         stk.sp = 0;
-        return T.n_tris != 0;
     }
-
-    __device__ __forceinline__ bool exhausted() const { return pend == 0 && node < 0 && stk.sp == 0; }
-
-    // One step; returns true when the walk has ended (found / best_* final,
-    // or for ANY a blocker found: found = true).
     __device__ __forceinline__ bool step(const Traversal& T, uint32_t& nvis, uint32_t& ntri) {
-        if (WIDTH == 2) return step2(T, nvis, ntri);
-        if (pend) {
-            const int k = __builtin_ctz(pend);  // nearest pending leaf
-            pend &= pend - 1u;
-            const int ref = (int)sel4(k, (uint32_t)pr0, (uint32_t)pr1, (uint32_t)pr2, (uint32_t)pr3);
-            const float tn = __uint_as_float(sel4(k, __float_as_uint(pk0), __float_as_uint(pk1),
-                                                  __float_as_uint(pk2), __float_as_uint(pk3)));
-            if (ANY || tn <= best_t) {
-                if (test_leaf<ANY, INSTR>(T, ref, o, d, best_t, best_s, best_o, found, ntri)) {
-                    found = true;
-                    return true;
-                }
-            }
-            return exhausted();
-        }
-        if (node < 0) node = stk.pop();  // not exhausted: the stack holds a node
-        if (INSTR) ++nvis;
-        const Bvh4Node* N = T.nodes4 + node;
-        const uint4 og = ldg(&N->org), qa = ldg(&N->qa), qb = ldg(&N->qb);
-        int4 rf = ldg(&N->ref);
-        // decode the quantised child boxes: org + q * 2^(e - 127).  The
-        // product is exact (q < 2^8, the scale a power of two, q * s normal or
-        // 0), so one fused multiply-add rounds to the same float as the
-        // host's multiply then add.
-        const float ox = __uint_as_float(og.x), oy = __uint_as_float(og.y), oz = __uint_as_float(og.z);
-        const float sx = __uint_as_float((og.w & 0xFFu) << 23), sy = __uint_as_float(((og.w >> 8) & 0xFFu) << 23),
-                    sz = __uint_as_float(((og.w >> 16) & 0xFFu) << 23);
-        float lxa[4], hxa[4], lya[4], hya[4], lza[4], hza[4];
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            lxa[k] = __builtin_fmaf((float)((qa.x >> (8 * k)) & 0xFFu), sx, ox);
-            hxa[k] = __builtin_fmaf((float)((qa.y >> (8 * k)) & 0xFFu), sx, ox);
-            lya[k] = __builtin_fmaf((float)((qa.z >> (8 * k)) & 0xFFu), sy, oy);
-            hya[k] = __builtin_fmaf((float)((qa.w >> (8 * k)) & 0xFFu), sy, oy);
-            lza[k] = __builtin_fmaf((float)((qb.x >> (8 * k)) & 0xFFu), sz, oz);
-            hza[k] = __builtin_fmaf((float)((qb.y >> (8 * k)) & 0xFFu), sz, oz);
-        }
-        int r[4] = {rf.x, rf.y, rf.z, rf.w};
-        float key[4];
-        const float lim = ANY ? 1.0f : best_t;
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            float tn, tf;
-            slab(sr, lxa[k], lya[k], lza[k], hxa[k], hya[k], hza[k], tn, tf);
-            const bool h = tn <= tf && tf >= 0.0f && tn <= lim && r[k] != kEmpty4;
-            key[k] = h ? tn : INFINITY;
-        }
-        // nearest first
-        cswap(key[0], r[0], key[1], r[1]);
-        cswap(key[2], r[2], key[3], r[3]);
-        cswap(key[0], r[0], key[2], r[2]);
-        cswap(key[1], r[1], key[3], r[3]);
-        cswap(key[1], r[1], key[2], r[2]);
-        // leaves become pending (tested nearest first)
-        pr0 = r[0];
-        pr1 = r[1];
-        pr2 = r[2];
-        pr3 = r[3];
-        pk0 = key[0];
-        pk1 = key[1];
-        pk2 = key[2];
-        pk3 = key[3];
-#pragma unroll
-        for (int k = 0; k < 4; ++k) pend |= (key[k] != INFINITY && r[k] < 0) ? (1u << k) : 0u;
-        // internal children: the nearest is visited next, the others pushed
-        // farthest first
-        node = -1;
-#pragma unroll
-        for (int k = 3; k >= 0; --k) {
-            if (key[k] == INFINITY || r[k] < 0) continue;
-            if (node >= 0) stk.push(node);
-            node = r[k];
-        }
-        return exhausted();
-    }
-
-    __device__ __forceinline__ bool step2(const Traversal& T, uint32_t& nvis, uint32_t& ntri) {
-        if (node < 0) node = stk.pop();
+        if (idle()) return false;
+        if (node < 0) node = stk.pop();  // not ended: the stack holds a node
         if (INSTR) ++nvis;
         const BvhNode* N = T.nodes + node;
         float4 a = ldg(&N->a), b = ldg(&N->b), c = ldg(&N->c);
@@ -548,18 +471,16 @@ struct Walker {
         bool h0 = tn0 <= tf0 && tf0 >= 0.0f && tn0 <= lim;
         bool h1 = tn1 <= tf1 && tf1 >= 0.0f && tn1 <= lim;
         if (h0 && ch.x < 0) {
-            if (test_leaf<ANY, INSTR>(T, ch.x, o, d, best_t, best_s, best_o, found, ntri)) {
-                found = true;
-                return true;
-            }
+            test_leaf<ANY, INSTR>(T, ch.x, o, d, best_t, best_s, best_o, ntri);
             h0 = false;
         }
-        if (h1 && ch.y < 0) {
-            if (test_leaf<ANY, INSTR>(T, ch.y, o, d, best_t, best_s, best_o, found, ntri)) {
-                found = true;
-                return true;
-            }
+        if (h1 && ch.y < 0 && !(ANY && found())) {
+            test_leaf<ANY, INSTR>(T, ch.y, o, d, best_t, best_s, best_o, ntri);
             h1 = false;
+        }
+        if (ANY && found()) {
+            node = kIdle;
+            return true;
         }
         node = -1;
         if (h0 && h1) {
@@ -571,7 +492,191 @@ struct Walker {
         } else if (h1) {
             node = ch.y;
         }
-        return node < 0 && stk.sp == 0;
+        if (node >= 0 || stk.sp > 0) return false;
+        node = kIdle;
+        return true;
+    }
+};
+
+// 4-wide tree: cur is the node to visit or the leaf to test; a visit sorts
+// the node's hit children (inner or leaf) by entry distance, takes the nearest
+// and pushes the others farthest first.  What bounds it is the vector unit:
+// of its instructions only f32 add, mul and fma, 32-bit logic, shifts and
+// adds issue at two per clock and CU (measured 1.7), while min, max, compares,
+// conversions and selects issue at one.  So the boxes' planes are folded to
+// one multiply-add each, the near and far planes are chosen by the sign of
+// the direction for all four children at once instead of by min and max, and
+// a wave's step is either a node visit or a triangle test, for the lanes at
+// one (whichever more of the wave's walks are at), so that no step runs both
+// for a few lanes each.  Hall of 200k triangles, 3 x 10M rays: closest hit
+// 176 -> 128 ms and any hit 137 -> 92 ms per render (1.34e11 -> 7.8e10 vector
+// instructions); each lane's 16-byte piece of a node or triangle is an L1
+// access of its own, 72 per closest-hit query, and the L1 takes one per clock
+// and CU: that is now the closest-hit kernel's bound (1.0 measured).
+template <int LDS, int BLOCK, bool ANY, bool INSTR>
+struct Walker<LDS, BLOCK, 4, ANY, INSTR> {
+    static constexpr int kIdle = kEmpty4;  // above every node index
+    V3 o, d;
+    float ix, iy, iz;  // 1 / d
+    float best_t = 0.0f;
+    int best_s = -1;
+    uint32_t best_o = 0;
+    int cur = kIdle;  // >= 0: the node to visit; < 0: the leaf to test
+    Stack<LDS, BLOCK> stk;
+
+    __device__ __forceinline__ Walker(int* lds, int* gstack, uint32_t gtid, uint32_t gthreads)
+        : stk(lds, gstack, gtid, gthreads) {}
+    __device__ __forceinline__ bool idle() const { return cur == kIdle; }
+    __device__ __forceinline__ bool found() const { return best_s >= 0; }
+    // 1 / x to an ulp: the boxes' padding covers it
+    static __device__ __forceinline__ float inv(float x) {
+        return __builtin_amdgcn_rcpf(fabsf(x) > 1e-20f ? x : copysignf(1e-20f, x));
+    }
+    __device__ __forceinline__ void start(const Traversal& T, V3 o_, V3 d_, float t_max) {
+        o = o_;
+        d = d_;
+        ix = inv(d.x);
+        iy = inv(d.y);
+        iz = inv(d.z);
+        best_t = t_max;
+        best_s = -1;
+        best_o = 0;
+        cur = T.n_tris != 0 ? 0 : kIdle;
+        stk.sp = 0;
+    }
+
+    // a and b swapped if m is all ones
+    static __device__ __forceinline__ void swap_if(uint32_t m, uint32_t& a, uint32_t& b) {
+        const uint32_t t = (a ^ b) & m;
+        a ^= t;
+        b ^= t;
+    }
+    static __device__ __forceinline__ uint32_t sign_mask(float x) { return (uint32_t)((int)__float_as_uint(x) >> 31); }
+
+    // orders two (entry distance, child) pairs
+    static __device__ __forceinline__ void order(float& ka, int& va, float& kb, int& vb) {
+        const bool sw = kb < ka;
+        const float k0 = fminf(ka, kb), k1 = fmaxf(ka, kb);
+        const int v0 = sw ? vb : va, v1 = sw ? va : vb;
+        ka = k0;
+        kb = k1;
+        va = v0;
+        vb = v1;
+    }
+
+    __device__ __forceinline__ bool visit(const Traversal& T) {
+        const Bvh4Node* N = (const Bvh4Node*)((const char*)T.nodes4 + ((uint32_t)cur << 6));
+        const uint4 og = ldg(&N->org);
+        uint4 qa = ldg(&N->qa), qb = ldg(&N->qb);
+        const int4 rf = ldg(&N->ref);
+        // planes org + q 2^e against the ray, one multiply-add each:
+        // (2^e / d) q + (org - o) / d.  The rounding moves a plane by a few
+        // 2^-24 of |org - o| (the boxes are padded by 1e-5 of the scene) and a
+        // distance by a few 2^-24 of itself, which the widened exit covers;
+        // the triangle test decides the hit.
+        const float ax = __uint_as_float((og.w << 23) & 0x7F800000u) * ix,
+                    ay = __uint_as_float((og.w << 15) & 0x7F800000u) * iy,
+                    az = __uint_as_float((og.w << 7) & 0x7F800000u) * iz;
+        const float bx = (__uint_as_float(og.x) - o.x) * ix, by = (__uint_as_float(og.y) - o.y) * iy,
+                    bz = (__uint_as_float(og.z) - o.z) * iz;
+        swap_if(sign_mask(ix), qa.x, qa.y);  // near, far
+        swap_if(sign_mask(iy), qa.z, qa.w);
+        swap_if(sign_mask(iz), qb.x, qb.y);
+        int r[4] = {rf.x, rf.y, rf.z, rf.w};
+        float key[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const float nx = __builtin_fmaf((float)((qa.x >> (8 * k)) & 0xFFu), ax, bx);
+            const float fx = __builtin_fmaf((float)((qa.y >> (8 * k)) & 0xFFu), ax, bx);
+            const float ny = __builtin_fmaf((float)((qa.z >> (8 * k)) & 0xFFu), ay, by);
+            const float fy = __builtin_fmaf((float)((qa.w >> (8 * k)) & 0xFFu), ay, by);
+            const float nz = __builtin_fmaf((float)((qb.x >> (8 * k)) & 0xFFu), az, bz);
+            const float fz = __builtin_fmaf((float)((qb.y >> (8 * k)) & 0xFFu), az, bz);
+            const float tn = fmaxf(fmaxf(fmaxf(nx, ny), nz), 0.0f);
+            const float tf = fminf(fminf(fminf(fx, fy), fz) * 1.000001f, ANY ? 1.0f : best_t);
+            key[k] = (tn <= tf) & (r[k] != kEmpty4) ? tn : INFINITY;
+        }
+        if (!ANY) {
+            // nearest first
+            order(key[0], r[0], key[1], r[1]);
+            order(key[2], r[2], key[3], r[3]);
+            order(key[0], r[0], key[2], r[2]);
+            order(key[1], r[1], key[3], r[3]);
+            order(key[1], r[1], key[2], r[2]);
+            if (key[3] != INFINITY) stk.push(r[3]);
+            if (key[2] != INFINITY) stk.push(r[2]);
+            if (key[1] != INFINITY) stk.push(r[1]);
+            cur = key[0] != INFINITY ? r[0] : kIdle;
+        } else {
+            // any order: the last hit child is taken, the others pushed
+            cur = key[0] != INFINITY ? r[0] : kIdle;
+#pragma unroll
+            for (int k = 1; k < 4; ++k) {
+                if (key[k] == INFINITY) continue;
+                if (cur != kIdle) stk.push(cur);
+                cur = r[k];
+            }
+        }
+        return cur == kIdle;
+    }
+
+    // the leaf's next two triangles (leaves hold two by default), their six
+    // loads in flight together
+    __device__ __forceinline__ bool test(const Traversal& T, uint32_t& ntri) {
+        const uint32_t i = (uint32_t)cur & 0x00FFFFFFu;
+        const int more = (int)(((uint32_t)cur >> 24) & 0x7Fu);  // triangles after the first
+        const float4* tp = (const float4*)((const char*)T.tris + i * 48u);
+        const float4* tq = tp + (more ? 3 : 0);
+        const float4 t0 = ldg(tp), t1 = ldg(tp + 1), t2 = ldg(tp + 2);
+        const float4 u0 = ldg(tq), u1 = ldg(tq + 1), u2 = ldg(tq + 2);
+        if (INSTR) ntri += more ? 2u : 1u;
+        accept(i, V3{t0.x, t0.y, t0.z}, V3{t0.w, t1.x, t1.y}, V3{t1.z, t1.w, t2.x}, __float_as_uint(t2.y));
+        // (a leaf of one: the same triangle again, which changes nothing)
+        accept(i + (more ? 1u : 0u), V3{u0.x, u0.y, u0.z}, V3{u0.w, u1.x, u1.y}, V3{u1.z, u1.w, u2.x},
+               __float_as_uint(u2.y));
+        cur = more > 1 ? cur - (2 << 24) + 2 : kIdle;
+        if (ANY && found()) {
+            cur = kIdle;
+            stk.sp = 0;
+        }
+        return cur == kIdle;
+    }
+    // mt_intersect's steps without branches: a wave of walks that rarely agree
+    // runs every one anyway
+    __device__ __forceinline__ void accept(uint32_t i, V3 v0, V3 e1, V3 e2, uint32_t orig) {
+        const V3 pvec = cross(d, e2);
+        const float det = dot(e1, pvec);
+        const float inv_det = 1.0f / det;
+        const V3 tvec = sub(o, v0);
+        const float u = dot(tvec, pvec) * inv_det;
+        const V3 qvec = cross(tvec, e1);
+        const float v = dot(d, qvec) * inv_det;
+        const float t = dot(e2, qvec) * inv_det;
+        bool in = !((det > -0.00001f) & (det < 0.00001f)) & !(u < 0.0f) & !(u > 1.0f) & !(v < 0.0f) & !(u + v > 1.0f);
+        if (ANY) {
+            in &= (t > 1e-5f) & (t < 1.0f);
+            best_s = in ? 0 : best_s;
+        } else {
+            in &= (t > 0.001f) & ((t < best_t) | ((t == best_t) & (orig < best_o)));
+            best_t = in ? t : best_t;
+            best_s = in ? (int)i : best_s;
+            best_o = in ? orig : best_o;
+        }
+    }
+
+    __device__ __forceinline__ bool step(const Traversal& T, uint32_t& nvis, uint32_t& ntri) {
+        const uint64_t ml = __ballot(cur < 0), mn = __ballot((uint32_t)cur < (uint32_t)kIdle);
+        bool pops = false;
+        if (__popcll(ml) >= __popcll(mn)) {
+            if (cur < 0) pops = test(T, ntri);
+        } else if ((uint32_t)cur < (uint32_t)kIdle) {
+            if (INSTR) ++nvis;
+            pops = visit(T);
+        }
+        if (!pops) return false;
+        if (stk.sp == 0) return true;
+        cur = stk.pop();
+        return false;
     }
 };
 
@@ -580,13 +685,12 @@ template <int LDS, int BLOCK, int WIDTH, bool ANY, bool INSTR>
 __device__ bool traverse(const Traversal& T, V3 o, V3 d, float& best_t, int& best_s, uint32_t& best_o, int* lds,
                          uint32_t gtid, uint32_t& nvis, uint32_t& ntri) {
     Walker<LDS, BLOCK, WIDTH, ANY, INSTR> w(lds, T.gstack, gtid, T.gthreads);
-    if (!w.start(T, o, d, best_t)) return false;
-    while (!w.step(T, nvis, ntri)) {
-    }
+    w.start(T, o, d, best_t);
+    while (!w.idle()) w.step(T, nvis, ntri);
     best_t = w.best_t;
     best_s = w.best_s;
     best_o = w.best_o;
-    return w.found;
+    return w.found();
 }
 
 // ---------------------------------------------------------------------------
@@ -1332,48 +1436,31 @@ __global__ void __launch_bounds__(BLOCK) k_extend_f(const InstDev* __restrict__ 
     uint32_t nvis = 0, ntri = 0;
     Walker<LDS, BLOCK, WIDTH, false, INSTR> w(lds + threadIdx.x, gstack, gtid, gthreads);
     Traversal T = make_trav(inst[0], gstack, gthreads);
-    // a lane is walking (active), holds a finished hit not yet stored
-    // (pending) or is free; pending hits are stored together when the wave
-    // refills, so the 8-byte records of a claimed run land in its cache lines
-    // in a few bursts instead of one lane at a time
-    bool active = false, pending = false, exhausted = n == 0;
-    uint32_t slot = 0;
-    int2 hit = make_int2(0, -1);
-    uint32_t c_next = 0, c_end = 0;  // the wave's claimed entries [c_next, c_end)
-    uint32_t seg = ((blockIdx.x * BLOCK + threadIdx.x) >> 6) % fetch.n_seg;  // the wave's first segment
+    Claim claim(n, gtid, gridDim.x * blockDim.x, fetch);
+    uint32_t refill = fetch.refill;  // idle lanes that trigger a refill
+    // A finished hit is stored with the wave's others at its next refill, so
+    // that the 8-byte records of a claimed run reach their cache lines in a
+    // few bursts instead of one lane at a time.
+    uint32_t slot = 0xFFFFFFFFu;  // this lane's queue entry
     for (;;) {
-        uint64_t act = __ballot(active);
-        const uint32_t n_idle = 64u - (uint32_t)__popcll(act);
-        if (n_idle >= fetch.refill || act == 0) {
-            if (pending) {
-                hits[slot] = hit;
-                pending = false;
-            }
-            if (!exhausted) {
-                const uint32_t mine = take_entries(fetch, n, act, lane, c_next, c_end, exhausted, seg);
-                if (mine != 0xFFFFFFFFu) {
-                    slot = mine;
-                    const float4 o = q.o[mine], d = q.d[mine];
-                    if (BATCH) T = make_trav(inst[q.m[mine].w], gstack, gthreads);
-                    if (w.start(T, V3{o.x, o.y, o.z}, V3{d.x, d.y, d.z}, 1000000.0f))
-                        active = true;
-                    else
-                        hits[mine] = make_int2(__float_as_int(1000000.0f), -1);
+        const uint64_t idle = __ballot(w.idle());
+        if ((uint32_t)__popcll(idle) >= refill) {
+            const uint32_t mine = claim.take(fetch, idle, lane);
+            if (w.idle()) {
+                if (slot != 0xFFFFFFFFu) hits[slot] = make_int2(__float_as_int(w.best_t), w.best_s);
+                slot = mine;
+                if (slot != 0xFFFFFFFFu) {
+                    const float4 o = q.o[slot], d = q.d[slot];
+                    if (BATCH) T = make_trav(inst[q.m[slot].w], gstack, gthreads);
+                    w.start(T, V3{o.x, o.y, o.z}, V3{d.x, d.y, d.z}, 1000000.0f);
                 }
             }
-            act = __ballot(active);
+            // the loop is left by the whole wave at once, with no walk and no
+            // hit left; with nothing left to take the next look is at the end
+            if (__ballot(slot != 0xFFFFFFFFu) == 0) break;
+            if (claim.exhausted()) refill = 64u;
         }
-        // the loop is left by the whole wave at once, with no hit pending
-        // (the refill step above has just stored them)
-        if (act == 0) {
-            if (exhausted) break;
-            continue;
-        }
-        if (active && w.step(T, nvis, ntri)) {
-            hit = make_int2(__float_as_int(w.best_t), w.best_s);
-            pending = true;
-            active = false;
-        }
+        w.step(T, nvis, ntri);
     }
     if (INSTR) {
         stat_add(stats, ST_NV_CL, nvis);
@@ -1432,52 +1519,37 @@ __global__ void __launch_bounds__(BLOCK, 6) k_shadow_f(const InstDev* __restrict
             ++ncon;
         }
     };
-    bool active = false, exhausted = n == 0;
+    Claim claim(n, gtid, gridDim.x * blockDim.x, fetch);
+    uint32_t refill = fetch.refill;  // idle lanes that trigger a refill
     uint32_t slot = 0;
-    uint32_t c_next = 0, c_end = 0;  // the wave's claimed entries [c_next, c_end)
-    uint32_t seg = ((blockIdx.x * BLOCK + threadIdx.x) >> 6) % fetch.n_seg;  // the wave's first segment
     for (;;) {
         if (nq >= 64) drain(64);
-        uint64_t act = __ballot(active);
-        const uint32_t n_free = 64u - (uint32_t)__popcll(act);
-        if (n_free >= fetch.refill || act == 0) {
-            if (!exhausted) {
-                const uint32_t mine = take_entries(fetch, n, act, lane, c_next, c_end, exhausted, seg);
-                bool vis = false;
-                if (mine != 0xFFFFFFFFu) {
-                    slot = mine;
-                    ++nsh;
-                    const float4 pc = sq.p[mine], m = sq.m[mine];
-                    const uint32_t packed = __float_as_uint(m.y);
-                    const uint32_t id = BATCH ? __float_as_uint(m.z) : 0;
-                    if (BATCH) T = make_trav(inst[id], gstack, gthreads);
-                    const RecParams& R = inst[id].P.rec[packed & 0xFFu];
-                    const V3 p{pc.x, pc.y, pc.z};
-                    if (w.start(T, p, sub(V3{R.px, R.py, R.pz}, p), 0.0f))
-                        active = true;
-                    else
-                        vis = true;  // empty scene: visible
-                }
-                push(vis, slot);
+        const uint64_t idle = __ballot(w.idle());
+        if ((uint32_t)__popcll(idle) >= refill) {
+            const uint32_t mine = claim.take(fetch, idle, lane);
+            if (mine != 0xFFFFFFFFu) {
+                slot = mine;
+                ++nsh;
+                const float4 pc = sq.p[mine], m = sq.m[mine];
+                const uint32_t packed = __float_as_uint(m.y);
+                const uint32_t id = BATCH ? __float_as_uint(m.z) : 0;
+                if (BATCH) T = make_trav(inst[id], gstack, gthreads);
+                const RecParams& R = inst[id].P.rec[packed & 0xFFu];
+                const V3 p{pc.x, pc.y, pc.z};
+                w.start(T, p, sub(V3{R.px, R.py, R.pz}, p), 0.0f);
             }
-            act = __ballot(active);
-        }
-        // the loop is left by the whole wave at once (take_entries is a
-        // wave-wide step), after the waiting records
-        if (act == 0) {
-            if (exhausted) {
+            push(mine != 0xFFFFFFFFu && w.idle(), slot);  // empty scene: visible
+            // the loop is left by the whole wave at once, after the waiting
+            // records; with nothing left to take the next look is at the end
+            if (idle == ~0ull && __ballot(mine != 0xFFFFFFFFu) == 0) {
                 while (nq > 0) drain(nq < 64u ? nq : 64u);
                 break;
             }
-            continue;
+            if (claim.exhausted()) refill = 64u;
         }
-        bool vis = false;
-        if (active && w.step(T, nvis, ntri)) {
-            active = false;
-            vis = !w.found;
-            if (TILED && w.found) TileSink{to, slot * to.stride, 0}.close();  // occluded: no records
-        }
-        push(vis, slot);
+        const bool ended = w.step(T, nvis, ntri);
+        if (TILED && ended && w.found()) TileSink{to, slot * to.stride, 0}.close();  // occluded: no records
+        push(ended && !w.found(), slot);
     }
     stat_add(stats, ST_SHADOW, nsh);
     stat_add(stats, ST_CONTRIB, ncon);
@@ -2630,7 +2702,7 @@ ear_status run_batch(Ctx* c, uint32_t n_items, DeviceScene* const* scenes, const
     const bool timed = eager && !noalloc;
     const uint32_t refill = tu.refill ? tu.refill : 24u;
     const uint32_t fchunk = tu.fetch_chunk;  // 0: one entry per idle lane
-    const uint32_t nseg = tu.fetch_segments ? std::min<uint32_t>(tu.fetch_segments, kMaxSeg) : 64u;
+    const uint32_t nseg = tu.fetch_segments ? std::min<uint32_t>(tu.fetch_segments, kMaxSeg) : kSegDefault;
     const Fetch fq_e{segc.as<uint32_t>(), refill, fchunk, nseg},
         fq_s{segc.as<uint32_t>() + kMaxSeg * kSegStride, refill, fchunk, nseg};
     // one iteration; cur = the queue it consumes
@@ -3550,14 +3622,13 @@ __global__ void __launch_bounds__(kBlock) k_adj_vis(const InstDev* __restrict__ 
     for (int q = 0; q < kAdMaxMat; ++q) g_refl[q] = g_spec[q] = 0.0;
     uint32_t key = 0xFFFFFFFFu;  // instance of the accumulated partials
     int kband = -1;
-    bool active = false, pending = false, exhausted = n == 0;
+    Claim claim(n, gtid, gridDim.x * blockDim.x, fetch);
+    uint32_t refill = fetch.refill;
+    bool pending = false;  // a visible request not yet added
     uint32_t slot = 0;
-    uint32_t c_next = 0, c_end = 0;
-    uint32_t seg = (gtid >> 6) % fetch.n_seg;
     for (;;) {
-        uint64_t act = __ballot(active);
-        const uint32_t n_free = 64u - (uint32_t)__popcll(act);
-        if (n_free >= fetch.refill || act == 0) {
+        const uint64_t idle = __ballot(w.idle());
+        if ((uint32_t)__popcll(idle) >= refill) {
             if (pending) {
                 const uint4 m = aq.m[slot];
                 const uint32_t id = BATCH ? m.y : 0u;
@@ -3588,35 +3659,24 @@ __global__ void __launch_bounds__(kBlock) k_adj_vis(const InstDev* __restrict__ 
                 }
                 pending = false;
             }
-            if (!exhausted) {
-                const uint32_t mine = take_entries(fetch, n, act, lane, c_next, c_end, exhausted, seg);
-                if (mine != 0xFFFFFFFFu) {
-                    slot = mine;
-                    ++nsh;
-                    const float4 pw = aq.p[mine];
-                    const uint4 m = aq.m[mine];
-                    const uint32_t id = BATCH ? m.y : 0u;
-                    if (BATCH) T = make_trav(inst[id], gstack, gthreads);
-                    const RecParams& R = inst[id].P.rec[m.x & 0xFFu];
-                    const V3 p{pw.x, pw.y, pw.z};
-                    if (w.start(T, p, sub(V3{R.px, R.py, R.pz}, p), 0.0f))
-                        active = true;
-                    else
-                        pending = true;  // empty scene: visible
-                }
+            const uint32_t mine = claim.take(fetch, idle, lane);
+            if (mine != 0xFFFFFFFFu) {
+                slot = mine;
+                ++nsh;
+                const float4 pw = aq.p[mine];
+                const uint4 m = aq.m[mine];
+                const uint32_t id = BATCH ? m.y : 0u;
+                if (BATCH) T = make_trav(inst[id], gstack, gthreads);
+                const RecParams& R = inst[id].P.rec[m.x & 0xFFu];
+                const V3 p{pw.x, pw.y, pw.z};
+                w.start(T, p, sub(V3{R.px, R.py, R.pz}, p), 0.0f);
+                pending = w.idle();  // empty scene: visible
             }
-            act = __ballot(active);
+            // the loop is left by the whole wave at once
+            if (idle == ~0ull && __ballot(mine != 0xFFFFFFFFu) == 0) break;
+            if (claim.exhausted()) refill = 64u;
         }
-        // the loop is left by the whole wave at once (take_entries is a
-        // wave-wide step)
-        if (act == 0) {
-            if (exhausted && __ballot(pending) == 0) break;
-            continue;
-        }
-        if (active && w.step(T, nvis, ntri)) {
-            active = false;
-            pending = !w.found;
-        }
+        if (w.step(T, nvis, ntri)) pending = !w.found();
     }
     stat_add(stats, ST_SHADOW, nsh);
     if (!BATCH) {
@@ -3812,7 +3872,7 @@ ear_status run_backward_batch(Ctx* c, uint32_t n_items, DeviceScene* const* scen
     DevBuf segc(c);
     TRY(segc.alloc(kMaxSeg * kSegStride * 4));
     EAR_HIP_TRY(c, hipMemsetAsync(segc.p, 0, segc.n, st));
-    const uint32_t nseg = tu.fetch_segments ? std::min<uint32_t>(tu.fetch_segments, kMaxSeg) : 64u;
+    const uint32_t nseg = tu.fetch_segments ? std::min<uint32_t>(tu.fetch_segments, kMaxSeg) : kSegDefault;
     const Fetch fq_e{segc.as<uint32_t>(), tu.refill ? tu.refill : 24u, tu.fetch_chunk, nseg};
     const uint32_t waves = tu.waves_per_cu ? tu.waves_per_cu : 32;
     const uint32_t cap_e = (uint32_t)c->num_cus * (uint32_t)std::max(1, resident_blocks((const void*)fe, 256));

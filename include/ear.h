@@ -379,7 +379,7 @@ typedef struct {
     uint32_t fetch_chunk;    /* refilling traversal: queue entries a wave claims per atomic
                                 (0: one per idle lane) */
     uint32_t fetch_segments; /* refilling traversal: queue segments with a claim counter each
-                                (1..64, default 64) */
+                                (1..64, default 16) */
     uint32_t tail_rays;      /* once every ray is emitted and at most this many are live,
                                 one launch traces each through all its remaining segments
                                 (same histograms); 0: default, 2^20, or every ray when no
