@@ -113,6 +113,8 @@ struct RenderParams {
     uint32_t n_band_slots;  // always 3 (histograms laid out per band slot)
     uint32_t band_mask;
     uint32_t hist_kinds;    // 1 signed, 2 signed + abs
+    uint32_t one_point;     // ramps are added as one point each (tracer.hip, OnePoint)
+    double ramp_slack;      // and the distance by which a ramp's bin may miss its own (m)
     int32_t src_kind;
     float src_pos[3];
     uint32_t src_n_tris;

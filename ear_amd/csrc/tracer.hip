@@ -42,6 +42,8 @@ constexpr int kShadeBlock = 256;  // k_shade: its block-wide appends take one co
 // in flight it accepts
 constexpr uint32_t kNoallocWaves = 16;
 constexpr size_t kNoallocMinRays = 4096;
+constexpr double kBinMetres = 343.0 / 44100.0;       // a histogram bin as a distance
+constexpr uint64_t kRawStage = 64ull * 1024 * 1024;  // bytes of raw sums staged at a time
 
 enum StatIdx {
     ST_SEGMENTS = 0,
@@ -696,12 +698,18 @@ __device__ bool traverse(const Traversal& T, V3 o, V3 d, float& best_t, int& bes
 // ---------------------------------------------------------------------------
 // histogram splat
 // ---------------------------------------------------------------------------
+// (global atomics: the accumulators' pointer comes out of a struct, and as a
+// generic one it would make flat atomics, which also wait for the LDS)
+typedef __attribute__((address_space(1))) unsigned long long GlobalU64;
+__device__ __forceinline__ unsigned long long add_global(unsigned long long* p, unsigned long long v) {
+    return __hip_atomic_fetch_add((GlobalU64*)p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
 __device__ __forceinline__ void acc128(unsigned long long* cell, I128 q) {
     unsigned long long lo = q.lo;
-    unsigned long long old = atomicAdd(cell, lo);
+    unsigned long long old = add_global(cell, lo);
     unsigned long long carry = (old + lo) < old ? 1ull : 0ull;
     unsigned long long hi = (unsigned long long)q.hi + carry;
-    if (hi) atomicAdd(cell + 1, hi);
+    if (hi) add_global(cell + 1, hi);
 }
 
 // Ramp of values (w - i) * A / w at bins s + i, i in [0, w), bins < 0 and
@@ -744,8 +752,20 @@ __device__ __forceinline__ RampPoints ramp_points(float A, int w, int ww) {
     return r;
 }
 
+// The one point of a ramp (see OnePoint): its slope, in two's complement
+__device__ __forceinline__ I128 ramp_slope(float A, int w) {
+    const double S = (double)A / (double)w;
+    const I128 q = fixed_from_double(S < 0.0 ? -S : S);
+    return S < 0.0 ? i128_neg(q) : q;
+}
+
 // The points of a clipped ramp (s0 < nb) added to row h with global atomics.
-__device__ __forceinline__ void splat_span(unsigned long long* h, uint32_t nb, uint32_t s0, int ww, int w, float A) {
+__device__ __forceinline__ void splat_span(unsigned long long* h, uint32_t nb, uint32_t one, uint32_t s0, int ww, int w,
+                                           float A) {
+    if (one) {
+        acc128(h + 2 * (size_t)(s0 + ((uint32_t)w & 1u) * nb), ramp_slope(A, w));
+        return;
+    }
     const RampPoints q = ramp_points(A, w, ww);
     unsigned long long* hp = q.neg ? h + 2 * (size_t)nb : h;  // gets +w*S and +S
     unsigned long long* hm = q.neg ? h : h + 2 * (size_t)nb;  // gets (w+1)*S
@@ -754,11 +774,11 @@ __device__ __forceinline__ void splat_span(unsigned long long* h, uint32_t nb, u
     if (s0 + (uint32_t)ww + 1 < nb) acc128(hp + 2 * (size_t)(s0 + ww + 1), q.sq);
 }
 
-__device__ uint32_t splat_ramp(unsigned long long* h, uint32_t nb, int s, int w, float A) {
+__device__ uint32_t splat_ramp(unsigned long long* h, uint32_t nb, uint32_t one, int s, int w, float A) {
     int ww;
     uint32_t cut;
     if (!ramp_span(nb, s, w, ww, cut)) return cut;
-    splat_span(h, nb, (uint32_t)s, ww, w, A);
+    splat_span(h, nb, one, (uint32_t)s, ww, w, A);
     return cut;
 }
 
@@ -800,14 +820,27 @@ struct TileOut {
 // ramps of c >= 0, row 1 the ramps of |c| for c < 0, so each contribution
 // updates one row; the finalize step turns them into signed = P - N and
 // |.| = P + N (exact: quantisation is odd-symmetric, the sums are integers).
+//
+// OnePoint: a ramp's width is the ceiling of the root of its distance, and its
+// bin is that distance over the speed of sound, moved by at most the head's
+// half delay: the distances that fall on one bin span less than a metre, and
+// their widths are one of two consecutive numbers.  So a row's two parts hold
+// the slopes of the ramps of even and of odd width that start at each bin, one
+// 128-bit add per ramp instead of three (a negative slope as its two's
+// complement), and k_finish, which knows from the bin which two widths they
+// are, sums the ramps into the bins they cover: the same integers.  Per pass
+// (adds skipped altogether in a copy): 32 rooms 36 of 198 ms, the 1M-ray box 6
+// of 40, a room with an emitting mesh 10 of 54 went to the three adds.
+// Without it (a head of nearly half a metre, or bins too late for binary32
+// distances: make_params) the parts are the "+" and "-" of second differences.
 struct Hist {
-    unsigned long long* cells;  // [band slot][channel][kind][+/-][bin] x {lo, hi}
-    uint32_t n_bins, n_ch, kinds;
+    unsigned long long* cells;  // [band slot][channel][kind][part][bin] x {lo, hi}
+    uint32_t n_bins, n_ch, kinds, one;
     uint32_t key_base, n_tiles;  // the time-tiled splat's keys of this render
     __device__ uint32_t row_index(int band, int ch, int kind) const {
         return ((uint32_t)band * n_ch + (uint32_t)ch) * kinds + (uint32_t)kind;
     }
-    // the row's "+" part; its "-" part follows at + 2 * n_bins
+    // the row's first part; its second follows at + 2 * n_bins
     __device__ unsigned long long* row(int band, int ch, int kind) const {
         return cells + 4 * (size_t)n_bins * row_index(band, ch, kind);
     }
@@ -829,7 +862,7 @@ struct TileSink {
 __device__ __forceinline__ void put_ramp(const Hist& H, int band, int ch, int kind, int s, int w, float A, Drops& dr,
                                          TileSink& sink, bool tiled) {
     if (!tiled) {
-        dr.add(splat_ramp(H.row(band, ch, kind), H.n_bins, s, w, A));
+        dr.add(splat_ramp(H.row(band, ch, kind), H.n_bins, H.one, s, w, A));
         return;
     }
     int ww;
@@ -838,7 +871,7 @@ __device__ __forceinline__ void put_ramp(const Hist& H, int band, int ch, int ki
     dr.add(cut);
     if (!any) return;
     if (w > kTileMaxW) {
-        splat_span(H.row(band, ch, kind), H.n_bins, (uint32_t)s, ww, w, A);
+        splat_span(H.row(band, ch, kind), H.n_bins, H.one, (uint32_t)s, ww, w, A);
         return;
     }
     const uint32_t i = sink.base + sink.used++;
@@ -978,7 +1011,7 @@ __device__ __forceinline__ Traversal make_trav(const InstDev& I, int* gstack, ui
     return Traversal{I.nodes, I.nodes4, I.tris, I.n_tris, gstack, gthreads};
 }
 __device__ __forceinline__ Hist make_hist(const InstDev& I) {
-    return Hist{I.hist, I.P.n_bins, I.P.n_channels, I.P.hist_kinds, I.key_base, I.n_tiles};
+    return Hist{I.hist, I.P.n_bins, I.P.n_channels, I.P.hist_kinds, I.P.one_point, I.key_base, I.n_tiles};
 }
 
 // ---------------------------------------------------------------------------
@@ -1140,11 +1173,11 @@ __device__ __forceinline__ void surface_hit(const InstDev& In, const RenderParam
     V3 o{ro.x, ro.y, ro.z};
     d = V3{rd.x, rd.y, rd.z};
     p = V3{o.x + d.x * t, o.y + d.y * t, o.z + d.z * t};
-    float4 nmv = In.nm[h.y];
+    float4 nmv = ldg(In.nm + h.y);
     V3 N{nmv.x, nmv.y, nmv.z};
     nrm = dot(N, d) > 0.0f ? V3{N.x * -1.0f, N.y * -1.0f, N.z * -1.0f} : N;
     uint32_t mat = __float_as_uint(nmv.w);
-    float4 mb = In.mat_band[3 * mat + band];  // {fl2 | -1, spec, retention, -}
+    float4 mb = ldg(In.mat_band + 3 * mat + band);  // {fl2 | -1, spec, retention, -}
     rng.init(P.seed, rm.x, P.ctx_word[band], P.instance, rm.y);
     bt = kReflect;
     if (mb.x >= 0.0f) bt = (rng.next() <= mb.x) ? kReflect : kRefract;
@@ -1232,7 +1265,7 @@ __global__ void __launch_bounds__(kShadeBlock, 6) k_shade(const InstDev* __restr
             if (In.log_hits && rm.x < P.trace_rays) {
                 if (k - 1 < P.trace_segs)
                     In.log_hits[((size_t)band * P.trace_rays + rm.x) * P.trace_segs + (k - 1)] =
-                        h.y >= 0 ? (int32_t)__float_as_uint(In.tris[3 * h.y + 2].y) : -1;
+                        h.y >= 0 ? (int32_t)__float_as_uint(ldg(In.tris + 3 * h.y + 2).y) : -1;
                 In.log_nseg[(size_t)band * P.trace_rays + rm.x] = k;
             }
             if (h.y >= 0) surface_hit(In, P, band, ro, rd, rm, h, rng, p, nrm, prev, d, I, L, spec, seg, bt, alive);
@@ -1666,7 +1699,7 @@ __global__ void __launch_bounds__(1024) k_tile_scan(uint32_t* __restrict__ cnt, 
 // kbase <= k (kbase ascending, kbase[n_items] = K).
 struct TileRow {
     unsigned long long* row;
-    uint32_t nb, t0;
+    uint32_t nb, t0, one;
 };
 __device__ __forceinline__ TileRow tile_row(const InstDev* __restrict__ inst, const uint32_t* __restrict__ kbase,
                                             uint32_t n_items, uint32_t k) {
@@ -1681,12 +1714,12 @@ __device__ __forceinline__ TileRow tile_row(const InstDev* __restrict__ inst, co
     const InstDev& In = inst[lo];
     const uint32_t rel = k - kbase[lo];
     const uint32_t nb = In.P.n_bins;
-    return TileRow{In.hist + 4 * (size_t)nb * (rel / In.n_tiles), nb, (rel % In.n_tiles) * kTile};
+    return TileRow{In.hist + 4 * (size_t)nb * (rel / In.n_tiles), nb, (rel % In.n_tiles) * kTile, In.P.one_point};
 }
 
 // A record's ramp added to HBM directly.
 __device__ __forceinline__ void splat_record(const TileRow& r, uint2 p) {
-    splat_span(r.row, r.nb, r.t0 + (p.y & 0xFFFFu), (int)((p.y >> 16) & 0xFFu), (int)(p.y >> 24), __uint_as_float(p.x));
+    splat_span(r.row, r.nb, r.one, r.t0 + (p.y & 0xFFFFu), (int)((p.y >> 16) & 0xFFu), (int)(p.y >> 24), __uint_as_float(p.x));
 }
 
 // Records of crowded keys to out[] grouped by key: a block recounts its share
@@ -1821,6 +1854,10 @@ __global__ void __launch_bounds__(kTileBlock) k_tile_splat(const InstDev* __rest
                     const uint2 p = pv[j];
                     const uint32_t o = p.y & 0xFFFFu;
                     const int ww = (int)((p.y >> 16) & 0xFFu), w = (int)(p.y >> 24);
+                    if (tr.one) {
+                        lds_acc128(acc + ((uint32_t)w & 1u) * 2 * kSpan, o, ramp_slope(__uint_as_float(p.x), w));
+                        continue;
+                    }
                     const RampPoints q = ramp_points(__uint_as_float(p.x), w, ww);
                     unsigned long long* tp = acc + (q.neg ? 2 * kSpan : 0u);  // gets +w*S and +S
                     unsigned long long* tm = acc + (q.neg ? 0u : 2 * kSpan);  // gets (w+1)*S
@@ -1984,9 +2021,28 @@ __global__ void __launch_bounds__(kFinBlock) k_finalize(const InstDev* __restric
     }
 }
 
+// The finished track of one bin from its signed (and |.|) sums: 2^-80, 1/N, the
+// direct sound (src/Scene.cpp:299-311) and gain^2 (src/Scene.cpp:313-316).
+__device__ __forceinline__ void finished_values(const InstDev& In, int band, uint32_t ch, uint32_t j, const I128 v[2]) {
+    if (!In.value) return;
+    const uint32_t nb = In.P.n_bins, n_ch = In.P.n_channels, kinds = In.P.hist_kinds;
+    const size_t r0 = (((size_t)band * n_ch + ch) * kinds) * nb;  // value rows
+    const DirectRamp dr = In.direct[(size_t)band * n_ch + ch];
+    const double S = dr.visible ? (double)dr.a / (double)dr.w : 0.0;
+    for (uint32_t kind = 0; kind < kinds; ++kind) {
+        double x = (double)v[kind].hi * 18446744073709551616.0 + (double)v[kind].lo;
+        x = x * 0x1p-80;  // 2^-EAR_FRAC_BITS
+        x = x * In.inv_n;
+        if (dr.visible && (int)j >= dr.s && (int)j < dr.s + dr.w) {
+            const double dv = (double)(dr.w - ((int)j - dr.s)) * S;
+            x += kind == 1 ? fabs(dv) : dv;
+        }
+        In.value[r0 + (size_t)kind * nb + j] = x * In.gain2;
+    }
+}
+
 // Per (instance, band, channel) and bin: the sign-split rows (if any) become
-// the signed and |.| sums, then the finished track: 2^-80, 1/N, the direct
-// sound (src/Scene.cpp:299-311) and gain^2 (src/Scene.cpp:313-316).
+// the signed and |.| sums, then the finished track.
 __global__ void __launch_bounds__(256) k_values(const InstDev* __restrict__ inst, const uint4* __restrict__ rows) {
     const uint4 rw = rows[blockIdx.y];
     const InstDev& In = inst[rw.x];
@@ -2009,19 +2065,66 @@ __global__ void __launch_bounds__(256) k_values(const InstDev* __restrict__ inst
         c1[2 * j] = v[1].lo;
         c1[2 * j + 1] = (unsigned long long)v[1].hi;
     }
-    if (!In.value) return;
-    const DirectRamp dr = In.direct[(size_t)band * n_ch + ch];
-    const double S = dr.visible ? (double)dr.a / (double)dr.w : 0.0;
-    for (uint32_t kind = 0; kind < kinds; ++kind) {
-        double x = (double)v[kind].hi * 18446744073709551616.0 + (double)v[kind].lo;
-        x = x * 0x1p-80;  // 2^-EAR_FRAC_BITS
-        x = x * In.inv_n;
-        if (dr.visible && (int)j >= dr.s && (int)j < dr.s + dr.w) {
-            const double dv = (double)(dr.w - ((int)j - dr.s)) * S;
-            x += kind == 1 ? fabs(dv) : dv;
+    finished_values(In, band, ch, j, v);
+}
+
+// One-point rows (see OnePoint) finished: per (instance, band, channel) and
+// bin, the ramps that cover the bin, ramps of width w that start at s adding
+// (w - (bin - s)) times their slopes' sum; then signed and |.| sums and the
+// finished track as in k_values.  Each bin looks back over the widths of its
+// own distance (33 bins at 3 s), so bins are independent: a grid over all of
+// them, where the prefix sums of k_finalize are one block per row (the hall's
+// 3 s stereo rows: 1.05 ms with 12 blocks, 0.1 ms here).  The rows must not be
+// written meanwhile: raw sums go to `raw` ([row][kind][bin], or null), rows
+// [row0, row0 + gridDim.y) of the table.
+__global__ void __launch_bounds__(256) k_finish(const InstDev* __restrict__ inst, const uint4* __restrict__ rows,
+                                                uint32_t row0, unsigned long long* __restrict__ raw,
+                                                const uint64_t* __restrict__ raw_off) {
+    const uint32_t row = row0 + blockIdx.y;
+    const uint4 rw = rows[row];
+    const InstDev& In = inst[rw.x];
+    const RenderParams& P = In.P;
+    const int band = (int)rw.y;
+    const uint32_t ch = rw.z, nb = P.n_bins, n_ch = P.n_channels, kinds = P.hist_kinds;
+    const uint32_t j = blockIdx.x * 256 + threadIdx.x;
+    if (j >= nb) return;
+    const size_t r0 = (((size_t)band * n_ch + ch) * kinds) * nb;
+    const ulonglong2* c0 = (const ulonglong2*)(In.hist + 4 * r0);  // [kind][parity][bin]
+    // the two widths of ramps that start at s are wl and wl + 1: the least
+    // distance of a ramp on bin s is s kBinMetres - slack
+    const double slack = P.ramp_slack;
+    const double d0 = (double)j * kBinMetres - slack;
+    int wl = d0 > 1.0 ? (int)ceil(sqrt(d0)) : 1;
+    I128 sum[2] = {I128{0, 0}, I128{0, 0}};
+    for (uint32_t i = 0; i <= j && (int)i <= wl; ++i) {
+        const uint32_t s = j - i;
+        const double d = (double)s * kBinMetres - slack;
+        while (wl > 1 && d <= (double)((wl - 1) * (wl - 1))) --wl;
+        if ((int)i > wl) break;  // (widths fall with s: no earlier ramp reaches this bin)
+        const uint32_t pe = (uint32_t)wl & 1u;  // the part of width wl; the other one holds wl + 1
+        for (uint32_t k = 0; k < kinds; ++k) {
+            const ulonglong2* h = c0 + (size_t)k * 2 * nb;
+            const ulonglong2 a = h[(size_t)pe * nb + s], b = h[(size_t)(pe ^ 1u) * nb + s];
+            // slopes are signed only where there is one kind
+            const auto scaled = [](ulonglong2 v, uint32_t m) {
+                const I128 q{v.x, (int64_t)v.y};
+                return q.hi < 0 ? i128_neg(i128_mul_small(i128_neg(q), m)) : i128_mul_small(q, m);
+            };
+            if (a.x | a.y) sum[k] = i128_add(sum[k], scaled(a, (uint32_t)(wl - (int)i)));
+            if (b.x | b.y) sum[k] = i128_add(sum[k], scaled(b, (uint32_t)(wl + 1 - (int)i)));
         }
-        In.value[r0 + (size_t)kind * nb + j] = x * In.gain2;
     }
+    I128 v[2] = {sum[0], I128{0, 0}};
+    if (kinds > 1) {
+        v[0] = i128_add(sum[0], i128_neg(sum[1]));
+        v[1] = i128_add(sum[0], sum[1]);
+    }
+    if (raw)
+        for (uint32_t k = 0; k < kinds; ++k) {
+            ulonglong2* o = (ulonglong2*)raw + raw_off[row] - raw_off[row0] + (size_t)k * nb + j;
+            *o = make_ulonglong2(v[k].lo, (unsigned long long)v[k].hi);
+        }
+    finished_values(In, band, ch, j, v);
 }
 
 // batched queries for tests and host tools
@@ -2219,6 +2322,22 @@ ear_status make_params(Ctx* c, const ear_render_desc* D, RenderParams* P) {
     P->n_band_slots = 3;
     P->band_mask = D->band_mask;
     P->hist_kinds = (D->flags & EAR_FLAG_ABS_HIST) ? 2 : 1;
+    // one point per ramp: a bin's ramps must have one of two consecutive
+    // widths, so the distances of one bin must span less than a metre: its own
+    // 343 / 44100 m, the head's delay either way, and the rounding of binary32
+    // times (2^-24 of the distance each; 1e-6 of the longest, and 1 mm)
+    double head = 0.0;
+    if (D->estimator == EAR_EST_NEE)
+        for (uint32_t r = 0; r < D->n_recorders; ++r) {
+            const ear_recorder& R = D->recorders[r];
+            if (R.kind != EAR_REC_STEREO) continue;
+            const double e = std::sqrt((double)R.right_ear[0] * R.right_ear[0] + (double)R.right_ear[1] * R.right_ear[1] +
+                                       (double)R.right_ear[2] * R.right_ear[2]);
+            const double h = std::fabs((double)R.head_size) * e;
+            head = h >= head ? h : (h < head ? head : 1e30);  // NaN: not one point
+        }
+    P->ramp_slack = head + 1e-3 + 1e-6 * kBinMetres * (double)D->hist_bins;
+    P->one_point = 2.0 * P->ramp_slack + kBinMetres < 0.98 ? 1u : 0u;
     P->src_kind = D->source.kind;
     for (int k = 0; k < 3; ++k) P->src_pos[k] = D->source.pos[k];
     P->flags = D->flags;
@@ -2346,7 +2465,7 @@ ear_status run_batch(Ctx* c, uint32_t n_items, DeviceScene* const* scenes, const
     size_t hist_cells = 0, value_cells = 0, direct_cells = 0, log_hits = 0, log_nseg = 0;
     std::vector<size_t> hist_off(n_items), value_off(n_items), direct_off(n_items), logh_off(n_items),
         logn_off(n_items);
-    bool any_value = false;
+    bool any_value = false, want_raw1 = false;
     size_t max_recs = 0;
     uint32_t any_mesh = 0;
     // time-tiled splat: keys (render, row, tile) of every render, and the
@@ -2392,6 +2511,11 @@ ear_status run_batch(Ctx* c, uint32_t n_items, DeviceScene* const* scenes, const
             I.P.src_n_tris = m;
             I.P.src_total_area = total;
         }
+        // raw sums of one-point rows are staged beside them: the no-allocation
+        // render's region has no room set aside for that
+        const bool raw1 = outs[i] && (outs[i]->raw || outs[i]->abs_raw);
+        if (noalloc && raw1) I.P.one_point = 0;
+        want_raw1 = want_raw1 || (raw1 && I.P.one_point);
         I.n_tiles = (I.P.n_bins + kTile - 1) / kTile;
         I.key_base = (uint32_t)std::min<uint64_t>(n_keys, 0xFFFFFFFFull);
         kbase[i] = I.key_base;
@@ -2479,7 +2603,7 @@ ear_status run_batch(Ctx* c, uint32_t n_items, DeviceScene* const* scenes, const
     DevBuf hits(c, ar), so(c, ar), sm(c, ar), counters(c, ar), stats(c, ar), hist(c, ar), gs(c, ar), direct(c, ar),
         value(c, ar), logh(c, ar), logn(c, ar), dinst(c, ar), dsegs(c, ar), dsegoff(c, ar), drows(c, ar),
         dvrows(c, ar), msrc(c, ar), segc(c, ar), tkey(c, ar), tpay(c, ar), tsort(c, ar), tcnt(c, ar), toff(c, ar),
-        tcur(c, ar), tkb(c, ar), tfirst(c, ar);
+        tcur(c, ar), tkb(c, ar), tfirst(c, ar), dorows(c, ar), dorawo(c, ar);
     // device memory that must start at a value: hipMemsetAsync, or in the
     // no-allocation render a fill kernel (no memset nodes if a caller
     // captures the stream)
@@ -2564,20 +2688,29 @@ ear_status run_batch(Ctx* c, uint32_t n_items, DeviceScene* const* scenes, const
     // the histogram rows of the finishing kernels: one per (instance, band,
     // channel, kind) for the prefix sums, one per (instance, band, channel)
     // for the combination step
-    std::vector<uint4> rows, vrows;
-    uint32_t max_nb = 1;
+    // (one-point items: one per (instance, band, channel), and where each row's
+    // raw sums begin, in cells)
+    std::vector<uint4> rows, vrows, orows;
+    std::vector<uint64_t> raw_off(1, 0);
+    uint32_t max_nb = 1, max_nb1 = 1;
     for (uint32_t i = 0; i < n_items; ++i)
         for (uint32_t b = 0; b < 3; ++b)
             if ((descs[i]->band_mask >> b) & 1u)
-                for (uint32_t ch = 0; ch < inst[i].P.n_channels; ++ch)
+                for (uint32_t ch = 0; ch < inst[i].P.n_channels; ++ch) {
+                    if (inst[i].P.one_point) {
+                        orows.push_back(make_uint4(i, b, ch, 0));
+                        raw_off.push_back(raw_off.back() + (uint64_t)inst[i].P.hist_kinds * inst[i].P.n_bins);
+                        max_nb1 = std::max(max_nb1, inst[i].P.n_bins);
+                        continue;
+                    }
                     for (uint32_t kind = 0; kind < inst[i].P.hist_kinds; ++kind) rows.push_back(make_uint4(i, b, ch, kind));
-    for (const uint4& r : rows)
-        if (r.w == 0) {
-            vrows.push_back(r);
-            max_nb = std::max(max_nb, inst[r.x].P.n_bins);
-        }
+                    vrows.push_back(make_uint4(i, b, ch, 0));
+                    max_nb = std::max(max_nb, inst[i].P.n_bins);
+                }
     TRY(drows.alloc(sizeof(uint4) * rows.size()));
     TRY(dvrows.alloc(sizeof(uint4) * vrows.size()));
+    TRY(dorows.alloc(sizeof(uint4) * orows.size()));
+    TRY(dorawo.alloc(8 * raw_off.size()));
 
     // the ray queues, their hit records and the shadow queue; a queue's
     // shading emits <= cap * recorders requests, and mesh sources add their
@@ -2839,10 +2972,57 @@ ear_status run_batch(Ctx* c, uint32_t n_items, DeviceScene* const* scenes, const
         k_direct<4><<<n_items, kBlock, 0, st>>>(di, gsp, gthreads, stp);
     else
         k_direct<2><<<n_items, kBlock, 0, st>>>(di, gsp, gthreads, stp);
-    EAR_HIP_TRY(c, hipMemcpyAsync(drows.p, rows.data(), sizeof(uint4) * rows.size(), hipMemcpyHostToDevice, st));
-    k_finalize<<<(uint32_t)rows.size(), kFinBlock, 0, st>>>(di, drows.as<uint4>());
-    EAR_HIP_TRY(c, hipMemcpyAsync(dvrows.p, vrows.data(), sizeof(uint4) * vrows.size(), hipMemcpyHostToDevice, st));
-    k_values<<<dim3((max_nb + 255) / 256, (uint32_t)vrows.size()), 256, 0, st>>>(di, dvrows.as<uint4>());
+    if (!rows.empty()) {
+        EAR_HIP_TRY(c, hipMemcpyAsync(drows.p, rows.data(), sizeof(uint4) * rows.size(), hipMemcpyHostToDevice, st));
+        k_finalize<<<(uint32_t)rows.size(), kFinBlock, 0, st>>>(di, drows.as<uint4>());
+        EAR_HIP_TRY(c, hipMemcpyAsync(dvrows.p, vrows.data(), sizeof(uint4) * vrows.size(), hipMemcpyHostToDevice, st));
+        k_values<<<dim3((max_nb + 255) / 256, (uint32_t)vrows.size()), 256, 0, st>>>(di, dvrows.as<uint4>());
+    }
+    // One-point rows: finished in one launch, or where raw sums are wanted in
+    // runs of rows whose sums fit a staging buffer (at most kRawStage, in the
+    // memory that the ray queues, now done with, gave back).
+    if (!orows.empty()) {
+        EAR_HIP_TRY(c, hipMemcpyAsync(dorows.p, orows.data(), sizeof(uint4) * orows.size(), hipMemcpyHostToDevice, st));
+        EAR_HIP_TRY(c, hipMemcpyAsync(dorawo.p, raw_off.data(), 8 * raw_off.size(), hipMemcpyHostToDevice, st));
+        const uint32_t n_or = (uint32_t)orows.size();
+        auto finish = [&](uint32_t r0, uint32_t n, unsigned long long* raw) {
+            for (uint32_t k = 0; k < n; k += 32768u)  // a grid's second dimension
+                k_finish<<<dim3((max_nb1 + 255) / 256, std::min(n - k, 32768u)), 256, 0, st>>>(
+                    di, dorows.as<uint4>(), r0 + k, raw ? raw + 2 * (raw_off[r0 + k] - raw_off[r0]) : nullptr,
+                    dorawo.as<uint64_t>());
+        };
+        if (!want_raw1) {
+            finish(0, n_or, nullptr);
+        } else {
+            EAR_HIP_TRY(c, hipStreamSynchronize(st));
+            for (DevBuf* b : {&qo[0], &qo[1], &qd[0], &qd[1], &qm[0], &qm[1], &hits, &so, &sm}) b->release();
+            uint64_t most = 0;
+            for (uint32_t r = 0; r < n_or; ++r) most = std::max(most, raw_off[r + 1] - raw_off[r]);
+            DevBuf stage(c);
+            const uint64_t cells = std::max(most, std::min<uint64_t>(raw_off[n_or], kRawStage / 16));
+            TRY(stage.alloc(cells * 16));
+            for (uint32_t r0 = 0; r0 < n_or;) {
+                uint32_t r1 = r0 + 1;
+                while (r1 < n_or && raw_off[r1 + 1] - raw_off[r0] <= cells) ++r1;
+                finish(r0, r1 - r0, stage.as<unsigned long long>());
+                EAR_HIP_TRY(c, hipGetLastError());
+                for (uint32_t r = r0; r < r1; ++r) {
+                    const uint4 w = orows[r];
+                    const RenderParams& P = inst[w.x].P;
+                    for (uint32_t k = 0; outs[w.x] && k < P.hist_kinds; ++k) {
+                        int64_t* raw = k == 0 ? outs[w.x]->raw : outs[w.x]->abs_raw;
+                        if (raw)
+                            EAR_HIP_TRY(c, hipMemcpyAsync(raw + 2 * ((size_t)w.y * P.n_channels + w.z) * P.n_bins,
+                                                          stage.as<unsigned long long>() +
+                                                              2 * (raw_off[r] - raw_off[r0] + (uint64_t)k * P.n_bins),
+                                                          (size_t)P.n_bins * 16, hipMemcpyDeviceToHost, st));
+                    }
+                }
+                EAR_HIP_TRY(c, hipStreamSynchronize(st));
+                r0 = r1;
+            }
+        }
+    }
     EAR_HIP_TRY(c, hipGetLastError());
     if (t1) EAR_HIP_TRY(c, hipEventRecord(t1, st));
     EAR_HIP_TRY(c, hipStreamSynchronize(st));
@@ -2862,7 +3042,7 @@ ear_status run_batch(Ctx* c, uint32_t n_items, DeviceScene* const* scenes, const
                     size_t ooff = ((size_t)b * nch + ch) * nb;
                     int64_t* raw = kind == 0 ? out->raw : out->abs_raw;
                     double* val = kind == 0 ? out->value : out->abs_value;
-                    if (raw)
+                    if (raw && !P.one_point)
                         EAR_HIP_TRY(c, hipMemcpyAsync(raw + 2 * ooff,
                                                       hist.as<unsigned long long>() + 2 * (hist_off[i] + 2 * roff),
                                                       nb * 16, hipMemcpyDeviceToHost, st));
@@ -3144,11 +3324,11 @@ __global__ void __launch_bounds__(kBlock) k_shade_ad(const InstDev* __restrict__
                 V3 o{ro.x, ro.y, ro.z};
                 V3 d{rd.x, rd.y, rd.z};
                 V3 p{o.x + d.x * t, o.y + d.y * t, o.z + d.z * t};
-                float4 nmv = In.nm[h.y];
+                float4 nmv = ldg(In.nm + h.y);
                 V3 N{nmv.x, nmv.y, nmv.z};
                 V3 nrm = dot(N, d) > 0.0f ? V3{N.x * -1.0f, N.y * -1.0f, N.z * -1.0f} : N;
                 uint32_t mat = __float_as_uint(nmv.w);
-                float4 mb = In.mat_band[3 * mat + band];
+                float4 mb = ldg(In.mat_band + 3 * mat + band);
                 Rng rng;
                 rng.init(P.seed, rm.x, P.ctx_word[band], P.instance, rm.y);
                 int bt = kReflect;
@@ -3439,11 +3619,11 @@ __global__ void __launch_bounds__(kBlock) k_shade_adl(const InstDev* __restrict_
                 const V3 o{ro.x, ro.y, ro.z};
                 const V3 d{rd.x, rd.y, rd.z};
                 p = V3{o.x + d.x * t, o.y + d.y * t, o.z + d.z * t};
-                const float4 nmv = In.nm[h.y];
+                const float4 nmv = ldg(In.nm + h.y);
                 const V3 N{nmv.x, nmv.y, nmv.z};
                 nrm = dot(N, d) > 0.0f ? V3{N.x * -1.0f, N.y * -1.0f, N.z * -1.0f} : N;
                 mat = __float_as_uint(nmv.w);
-                const float4 mb = In.mat_band[3 * mat + band];
+                const float4 mb = ldg(In.mat_band + 3 * mat + band);
                 if (contn) {
                     kspawn = __float_as_uint(tin.row(nm, i));
                     score_rng_init(rng, P.seed, rm.x, P.ctx_word[band], P.instance, kspawn, rm.y);
