@@ -143,6 +143,34 @@ __device__ __forceinline__ uint32_t block_append(uint32_t* counter, bool pred, u
     return sc[kWaves] + sc[wave] + (uint32_t)__popcll(mask & ((1ull << lane) - 1ull));
 }
 
+// Two appends of a block with one atomic: a wave's `a` entries to the counter
+// in the low word and `b` to the one in the high word of `counter` (neither
+// overflows: a queue holds fewer than 2^32).  Adds to one address take about
+// 12.5 ns each whoever makes them, so with one per block step and queue the
+// appends were k_shade's whole time.  Every thread of the block calls it with
+// its wave's counts; `sc`: scratch of BLOCK / 64 words that consecutive calls
+// must not share.  Returns the wave's first slots {a, b}.
+template <int BLOCK>
+__device__ __forceinline__ uint2 block_append2(unsigned long long* counter, uint32_t a, uint32_t b,
+                                               unsigned long long* sc) {
+    const uint32_t wave = threadIdx.x >> 6;
+    if (lane_id() == 0) sc[wave] = (unsigned long long)a | ((unsigned long long)b << 32);
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        unsigned long long tot = 0;
+        for (uint32_t w = 0; w < BLOCK / 64; ++w) tot += sc[w];
+        unsigned long long base = tot ? atomicAdd(counter, tot) : 0ull;
+        for (uint32_t w = 0; w < BLOCK / 64; ++w) {
+            const unsigned long long c = sc[w];
+            sc[w] = base;
+            base += c;
+        }
+    }
+    __syncthreads();
+    const unsigned long long mine = sc[wave];
+    return make_uint2((uint32_t)mine, (uint32_t)(mine >> 32));
+}
+
 // Orders one wave's LDS accesses (lanes read what other lanes of the same
 // wave wrote; the LDS executes a wave's instructions in order).
 __device__ __forceinline__ void wave_sync() {
@@ -162,6 +190,20 @@ __device__ __forceinline__ void wave_sync() {
 // block per candidate until its slowest lane accepts.  All lanes of the wave
 // call it; `need` marks those that sample: around normal n if `hemi`
 // (sample_hemi), else the whole sphere (sample_sphere).
+//
+// A candidate f of squared length l is in the hemisphere if dot(n, f / |f|) is
+// not negative.  Almost always dot(n, f) tells: the two differ by at most
+// 4.2e-7 |n| |f| in rounding (four and three roundings of 2^-24 each on terms
+// whose sum of sizes is at most |n| |f|), so past 1e-6 its sign is the
+// quotient's.  The root and three divisions are then left for the accepted
+// candidate, after the rounds.
+__device__ __forceinline__ bool upper(V3 n, V3 f, float l) {
+    const float a = dot(n, f);
+    if (a < -1e-6f) return false;
+    if (fabsf(a) > 1e-6f) return true;
+    const float s = sqrtf(l);
+    return !(dot(n, V3{f.x / s, f.y / s, f.z / s}) < 0.0f);
+}
 struct HemiLds {
     uint4 own[64];   // the rank-th sampling lane's ray, ctx, inst and first block to compute
     uint2 key[64];   // its Philox key
@@ -169,7 +211,8 @@ struct HemiLds {
 };
 __device__ __forceinline__ V3 sample_hemi_wave(bool need, bool hemi, Rng& rng, V3 n, HemiLds& S) {
     const uint32_t lane = lane_id();
-    V3 v{0.0f, 0.0f, 0.0f};
+    V3 v{0.0f, 0.0f, 0.0f};  // the accepted candidate and its squared length
+    float vl = 1.0f;
     uint64_t act = __ballot(need);
     while (act) {
         const uint32_t A = (uint32_t)__popcll(act);
@@ -207,10 +250,9 @@ __device__ __forceinline__ V3 sample_hemi_wave(bool need, bool hemi, Rng& rng, V
                 off += 3u;
                 const float l = f1 * f1 + f2 * f2 + f3 * f3;
                 if (l < 0.001f || l > 1.0f) continue;
-                const float s = sqrtf(l);
-                const V3 c{f1 / s, f2 / s, f3 / s};
-                if (hemi && dot(n, c) < 0.0f) continue;
-                v = c;
+                if (hemi && !upper(n, V3{f1, f2, f3}, l)) continue;
+                v = V3{f1, f2, f3};
+                vl = l;
                 left = false;
                 break;
             }
@@ -226,7 +268,8 @@ __device__ __forceinline__ V3 sample_hemi_wave(bool need, bool hemi, Rng& rng, V
         wave_sync();  // this round's reads before the next round's writes
         act = __ballot(left);
     }
-    return v;
+    const float s = sqrtf(vl);
+    return V3{v.x / s, v.y / s, v.z / s};
 }
 
 // Statistics counters: [kStatCopies][ST_N], a block adding into copy
@@ -1024,11 +1067,14 @@ template <bool BATCH>
 __global__ void __launch_bounds__(kBlock) k_generate(const InstDev* __restrict__ inst, const GenSeg* __restrict__ segs,
                                                       const uint32_t* __restrict__ seg_off, uint32_t n_segs,
                                                       uint32_t total, const uint32_t* __restrict__ plan,
-                                                      uint32_t max_rec, uint32_t any_mesh, Queue q,
+                                                      uint32_t max_rec, uint32_t any_mesh, uint32_t dense, Queue q,
                                                       uint32_t* __restrict__ n_q, ShadowQ sq,
                                                       uint32_t* __restrict__ n_sq, unsigned long long* __restrict__ stats) {
     // rays [first, first + total) of the segment table; a plan written on the
-    // device (k_plan) overrides the host's range
+    // device (k_plan) overrides the host's range.  dense: every ray is live, so
+    // ray i of the range has slot plan[2] + i and k_plan counts them (an
+    // append's atomic per wave, 12.5 ns each on one address, was this kernel's
+    // whole time: 5.7 ms of a 30M-ray render, 1.3 ms without)
     uint32_t first = 0;
     if (plan) {
         first = plan[0];
@@ -1119,7 +1165,7 @@ __global__ void __launch_bounds__(kBlock) k_generate(const InstDev* __restrict__
                 }
             }
         }
-        uint32_t slot = wave_append(n_q, live);
+        const uint32_t slot = dense ? plan[2] + base + threadIdx.x : wave_append(n_q, live);
         if (live) {
             q.o[slot] = ro;
             q.d[slot] = rd;
@@ -1229,10 +1275,9 @@ __device__ __forceinline__ bool nee_weight(const RenderParams& P, const RecParam
 template <bool BATCH>
 __global__ void __launch_bounds__(kShadeBlock, 6) k_shade(const InstDev* __restrict__ inst, Queue qin,
                                                    const uint32_t* __restrict__ n_in, const int2* __restrict__ hits,
-                                                   Queue qout, uint32_t* __restrict__ n_out, ShadowQ sq,
-                                                   uint32_t* __restrict__ n_sq, uint32_t max_rec,
-                                                   unsigned long long* __restrict__ stats) {
-    __shared__ uint32_t sc[4][kShadeBlock / 64 + 1];  // scratch of the block-wide appends, alternated
+                                                   Queue qout, ShadowQ sq, unsigned long long* __restrict__ n_out,
+                                                   uint32_t max_rec, unsigned long long* __restrict__ stats) {
+    __shared__ unsigned long long sc[2][kShadeBlock / 64];  // scratch of the block-wide appends, alternated
     __shared__ HemiLds hl[kShadeBlock / 64];
     uint32_t n = *n_in;
     uint32_t n_done = 0, n_sph = 0;
@@ -1276,38 +1321,49 @@ __global__ void __launch_bounds__(kShadeBlock, 6) k_shade(const InstDev* __restr
                 nee = false;
             }
         }
-        // NEE to every recorder (src/Scene.cpp:185-268)
-        for (uint32_t r = 0; r < max_rec; ++r) {
-            bool emit = false;
+        // NEE to every recorder (src/Scene.cpp:185-268).  The slots of the
+        // connections and of the continuing rays come from one append, so the
+        // connections are counted before they are stored; the first two
+        // recorders' weights are kept for that, the others' computed again.
+        auto weight = [&](uint32_t r, float& c) -> bool {
+            if (!(alive && nee && r < n_rec)) return false;
+            const RenderParams& P = inst[id].P;
+            return nee_weight(P, P.rec[r], band, p, nrm, prev, bt, spec, I, k, c);
+        };
+        if (alive) cont = !((double)I < inst[id].P.cutoff) && k < inst[id].P.max_bounces;
+        float c0 = 0.0f, c1 = 0.0f;
+        const bool e0 = max_rec > 0 && weight(0, c0), e1 = max_rec > 1 && weight(1, c1);
+        uint32_t n_con = (uint32_t)(__popcll(__ballot(e0)) + __popcll(__ballot(e1)));
+        for (uint32_t r = 2; r < max_rec; ++r) {
             float c = 0.0f;
-            if (alive && nee && r < n_rec) {
-                const RenderParams& P = inst[id].P;
-                emit = nee_weight(P, P.rec[r], band, p, nrm, prev, bt, spec, I, k, c);
-            }
-            uint32_t slot = block_append<kShadeBlock>(n_sq, emit, sc[r & 1u]);
+            n_con += (uint32_t)__popcll(__ballot(weight(r, c)));
+        }
+        const uint64_t mcont = __ballot(cont);
+        const uint64_t below = (1ull << lane_id()) - 1ull;
+        const uint2 first = block_append2<kShadeBlock>(n_out, (uint32_t)__popcll(mcont), n_con,
+                                                       sc[(base / (gridDim.x * kShadeBlock)) & 1u]);
+        uint32_t next = first.y;
+        for (uint32_t r = 0; r < max_rec; ++r) {
+            float c = r == 0 ? c0 : c1;
+            const bool emit = r == 0 ? e0 : r == 1 ? e1 : weight(r, c);
+            const uint64_t m = __ballot(emit);
             if (emit) {
+                const uint32_t slot = next + (uint32_t)__popcll(m & below);
                 sq.p[slot] = make_float4(p.x, p.y, p.z, c);
                 sq.m[slot] = make_float4(L, __uint_as_float(r | ((uint32_t)band << 8)), __uint_as_float(id), 0.0f);
             }
+            next += (uint32_t)__popcll(m);
         }
-        if (alive) cont = !((double)I < inst[id].P.cutoff) && k < inst[id].P.max_bounces;
-        float4 no{}, nd{};
-        uint4 nmeta{};
         const V3 hv = sample_hemi_wave(cont, true, rng, nrm, hl[threadIdx.x >> 6]);
         if (cont) {
             // REFRACT: the negated normal and the incoming direction; REFLECT:
             // the mirror direction about the ray-facing normal (src/Scene.cpp:65-74)
             V3 rdir = bt == kRefract ? d : reflect(d, nrm);
             V3 v = blend_spec(hv, rdir, spec);
-            no = make_float4(p.x, p.y, p.z, I);
-            nd = make_float4(v.x, v.y, v.z, L);
-            nmeta = make_uint4(rm.x, rng.draw, (uint32_t)band | (k << 8), id);
-        }
-        uint32_t slot = block_append<kShadeBlock>(n_out, cont, sc[2 + ((base / (gridDim.x * kShadeBlock)) & 1u)]);
-        if (cont) {
-            qout.o[slot] = no;
-            qout.d[slot] = nd;
-            qout.m[slot] = nmeta;
+            const uint32_t slot = first.x + (uint32_t)__popcll(mcont & below);
+            qout.o[slot] = make_float4(p.x, p.y, p.z, I);
+            qout.d[slot] = make_float4(v.x, v.y, v.z, L);
+            qout.m[slot] = make_uint4(rm.x, rng.draw, (uint32_t)band | (k << 8), id);
         }
         n_done += valid ? 1u : 0u;
     }
@@ -1892,16 +1948,19 @@ __global__ void k_reset2(uint32_t* a, uint32_t* b) {
 }
 
 // Ray regeneration: tops the current queue up to `cap` with the next rays of
-// the segment table.  plan = {first ray, count} for k_generate; the cursor
-// counts the rays taken so far.
-__global__ void k_plan(uint32_t* cursor, uint32_t total, uint32_t cap, const uint32_t* n_q, uint32_t* plan) {
+// the segment table.  plan = {first ray, count, first free slot} for
+// k_generate; the cursor counts the rays taken so far.  dense: the rays are
+// counted into the queue here (k_generate appends them otherwise).
+__global__ void k_plan(uint32_t* cursor, uint32_t total, uint32_t cap, uint32_t dense, uint32_t* n_q, uint32_t* plan) {
     if (threadIdx.x == 0 && blockIdx.x == 0) {
         const uint32_t taken = *cursor, live = *n_q;
         const uint32_t room = cap > live ? cap - live : 0u;
         const uint32_t take = min(room, total - taken);
         plan[0] = taken;
         plan[1] = take;
+        plan[2] = live;
         *cursor = taken + take;
+        if (dense) *n_q = live + take;
     }
 }
 
@@ -2619,8 +2678,7 @@ ear_status run_batch(Ctx* c, uint32_t n_items, DeviceScene* const* scenes, const
         EAR_HIP_TRY(c, hipGetLastError());
         return EAR_OK;
     };
-    // [0] queue 0, [1] queue 1, [2] shadow queue, [3] generation cursor,
-    // [6..7] plan {first, count}
+    // see iteration()
     TRY(counters.alloc(16 * 4));
     // refill counters of the closest-hit and shadow kernels, one per line
     TRY(segc.alloc(2 * kMaxSeg * kSegStride * 4));
@@ -2755,16 +2813,16 @@ ear_status run_batch(Ctx* c, uint32_t n_items, DeviceScene* const* scenes, const
         tile_out.pay = tpay.as<uint2>();
     }
 
-    uint32_t* cnt = counters.as<uint32_t>();  // [0],[1] ray queues, [2] shadow queue
+    uint32_t* cnt = counters.as<uint32_t>();
     unsigned long long* stp = stats.as<unsigned long long>();
     const InstDev* di = dinst.as<InstDev>();
     int* gsp = gs.as<int>();
 
     // the queue counters read by the host: pinned memory, or in the
     // no-allocation render a host array (a synchronous copy)
-    uint32_t host_cnt[4] = {0, 0, 0, 0};
+    uint32_t host_cnt[8] = {};
     uint32_t* pinned = host_cnt;
-    if (!noalloc) EAR_HIP_TRY(c, hipHostMalloc((void**)&pinned, 16, hipHostMallocDefault));
+    if (!noalloc) EAR_HIP_TRY(c, hipHostMalloc((void**)&pinned, 32, hipHostMallocDefault));
     struct PinGuard {
         uint32_t* p;
         ~PinGuard() {
@@ -2811,6 +2869,10 @@ ear_status run_batch(Ctx* c, uint32_t n_items, DeviceScene* const* scenes, const
     }
     const uint32_t n_segs = (uint32_t)std::max<size_t>(1, all.size());
     const uint32_t total32 = (uint32_t)total_rays;
+    // every emitted ray has a first segment to trace
+    uint32_t dense = 1;
+    for (uint32_t i = 0; i < n_items; ++i)
+        if (1.0 < inst[i].P.cutoff || inst[i].P.max_bounces == 0) dense = 0;
     const uint32_t g_gen = grid_for(
         cap_rays, rounds_cap(c, batch ? (const void*)k_generate<true> : (const void*)k_generate<false>, tu.waves_per_cu, kBlock),
         kBlock);
@@ -2840,16 +2902,18 @@ ear_status run_batch(Ctx* c, uint32_t n_items, DeviceScene* const* scenes, const
         fq_s{segc.as<uint32_t>() + kMaxSeg * kSegStride, refill, fchunk, nseg};
     // one iteration; cur = the queue it consumes
     auto iteration = [&](int cur) {
-        uint32_t* nq = cnt + cur;
-        k_plan<<<1, 64, 0, st>>>(cnt + 3, total32, cap_rays, nq, cnt + 6);
+        // [2 q] rays of queue q, [2 q + 1] the shadow requests made with it as
+        // the output queue; [4] generation cursor, [6..8] plan
+        uint32_t *nq = cnt + 2 * cur, *nsq = cnt + 2 * (1 - cur) + 1;
+        k_plan<<<1, 64, 0, st>>>(cnt + 4, total32, cap_rays, dense, nq, cnt + 6);
         if (batch)
             k_generate<true><<<g_gen, kBlock, 0, st>>>(di, dsegs.as<GenSeg>(), dsegoff.as<uint32_t>(), n_segs, 0u,
-                                                       cnt + 6, (uint32_t)max_recs, any_mesh, qq[cur], nq, SQ,
-                                                       cnt + 2, stp);
+                                                       cnt + 6, (uint32_t)max_recs, any_mesh, dense, qq[cur], nq, SQ,
+                                                       nsq, stp);
         else
             k_generate<false><<<g_gen, kBlock, 0, st>>>(di, dsegs.as<GenSeg>(), dsegoff.as<uint32_t>(), n_segs, 0u,
-                                                        cnt + 6, (uint32_t)max_recs, any_mesh, qq[cur], nq, SQ,
-                                                        cnt + 2, stp);
+                                                        cnt + 6, (uint32_t)max_recs, any_mesh, dense, qq[cur], nq, SQ,
+                                                        nsq, stp);
         EventPair* e1 = timed ? &mk(ev_ext) : nullptr;
         if (e1) hipEventRecord(e1->a, st);
         hipLaunchKernelGGL(fe, dim3(g_ext), dim3(cfg_e.block), 0, st, di, gsp, gthreads, qq[cur], (const uint32_t*)nq,
@@ -2857,28 +2921,29 @@ ear_status run_batch(Ctx* c, uint32_t n_items, DeviceScene* const* scenes, const
         if (e1) hipEventRecord(e1->b, st);
         EventPair* e2 = timed ? &mk(ev_sha) : nullptr;
         if (e2) hipEventRecord(e2->a, st);
+        unsigned long long* n_out = (unsigned long long*)(cnt + 2 * (1 - cur));
         if (batch)
-            k_shade<true><<<g_shade, kShadeBlock, 0, st>>>(di, qq[cur], nq, hits.as<int2>(), qq[1 - cur], cnt + (1 - cur),
-                                                      SQ, cnt + 2, (uint32_t)max_recs, stp);
+            k_shade<true><<<g_shade, kShadeBlock, 0, st>>>(di, qq[cur], nq, hits.as<int2>(), qq[1 - cur], SQ, n_out,
+                                                           (uint32_t)max_recs, stp);
         else
-            k_shade<false><<<g_shade, kShadeBlock, 0, st>>>(di, qq[cur], nq, hits.as<int2>(), qq[1 - cur],
-                                                       cnt + (1 - cur), SQ, cnt + 2, (uint32_t)max_recs, stp);
+            k_shade<false><<<g_shade, kShadeBlock, 0, st>>>(di, qq[cur], nq, hits.as<int2>(), qq[1 - cur], SQ, n_out,
+                                                            (uint32_t)max_recs, stp);
         if (e2) hipEventRecord(e2->b, st);
         EventPair* e3 = timed ? &mk(ev_shw) : nullptr;
         if (e3) hipEventRecord(e3->a, st);
-        hipLaunchKernelGGL(fs, dim3(g_shw), dim3(cfg_s.block), 0, st, di, gsp, gthreads, SQ, (const uint32_t*)(cnt + 2),
+        hipLaunchKernelGGL(fs, dim3(g_shw), dim3(cfg_s.block), 0, st, di, gsp, gthreads, SQ, (const uint32_t*)nsq,
                            stp, fq_s, tile_out);
         if (e3) hipEventRecord(e3->b, st);
         if (tiled) {
             // the records of this launch, grouped by key and splatted per tile
             EventPair* e4 = timed ? &mk(ev_spl) : nullptr;
             if (e4) hipEventRecord(e4->a, st);
-            k_tile_count<<<g_tile, kTileBlock, 0, st>>>(tkey.as<uint32_t>(), cnt + 2, tile_stride, tcnt.as<uint32_t>(),
+            k_tile_count<<<g_tile, kTileBlock, 0, st>>>(tkey.as<uint32_t>(), nsq, tile_stride, tcnt.as<uint32_t>(),
                                                         K);
             k_tile_scan<<<1, 1024, 0, st>>>(tcnt.as<uint32_t>(), toff.as<uint32_t>(), tcur.as<uint32_t>(), K,
                                             tfirst.as<uint32_t>());
             k_tile_scatter<<<g_tile, kTileBlock, 0, st>>>(di, tkb.as<uint32_t>(), n_items, tkey.as<uint32_t>(),
-                                                          tpay.as<uint2>(), cnt + 2, tile_stride, tcur.as<uint32_t>(),
+                                                          tpay.as<uint2>(), nsq, tile_stride, tcur.as<uint32_t>(),
                                                           K, tsort.as<uint2>());
             k_tile_splat<<<g_splat, kTileBlock, 0, st>>>(di, tkb.as<uint32_t>(), n_items, toff.as<uint32_t>(), K,
                                                          tfirst.as<uint32_t>(), tsort.as<uint2>());
@@ -2886,19 +2951,19 @@ ear_status run_batch(Ctx* c, uint32_t n_items, DeviceScene* const* scenes, const
             launches += 4;
         }
         // the consumed queue, the shadow queue and the fetch counters
-        k_reset_iter<<<1, 64, 0, st>>>(cnt, (1u << cur) | 0x4u, segc.as<uint32_t>(), 2 * kMaxSeg);
+        k_reset_iter<<<1, 64, 0, st>>>(cnt, (1u << (2 * cur)) | (1u << (2 * (1 - cur) + 1)), segc.as<uint32_t>(), 2 * kMaxSeg);
         launches += 6;
         ++bounces;
     };
     // the render has ended once every ray was taken and no queue holds any
     auto finished = [&](int cur, bool* done) -> ear_status {
-        EAR_HIP_TRY(c, hipMemcpyAsync(pinned, cnt, 16, hipMemcpyDeviceToHost, st));
+        EAR_HIP_TRY(c, hipMemcpyAsync(pinned, cnt, 20, hipMemcpyDeviceToHost, st));
         EAR_HIP_TRY(c, hipStreamSynchronize(st));
-        *done = pinned[cur] == 0 && pinned[3] == total32;
+        *done = pinned[2 * cur] == 0 && pinned[4] == total32;
         return EAR_OK;
     };
     // the tail: every ray emitted and few live ones left (queue cur, of
-    // pinned[cur] rays, read by finished); one launch traces them to their ends
+    // pinned[2 cur] rays, read by finished); one launch traces them to their ends
     // (tail_rays 0: 2^20 live rays, measured best on the 200k-triangle hall,
     // or every ray when no scene has more than 64 triangles: their walks are
     // so short that the queues between the wavefront kernels cost more than
@@ -2912,9 +2977,9 @@ ear_status run_batch(Ctx* c, uint32_t n_items, DeviceScene* const* scenes, const
     for (uint32_t i = 0; i < n_items; ++i) tail_ok = tail_ok && inst[i].P.estimator == EAR_EST_NEE;
     const TailFn ft = tail_ok ? pick_tail(cfg_e) : nullptr;
     auto tail = [&](int cur, bool* done) -> ear_status {
-        if (*done || !ft || pinned[3] != total32 || pinned[cur] > tail_rays) return EAR_OK;
+        if (*done || !ft || pinned[4] != total32 || pinned[2 * cur] > tail_rays) return EAR_OK;
         hipLaunchKernelGGL(ft, dim3(g_ext), dim3(cfg_e.block), 0, st, di, gsp, gthreads, qq[cur],
-                           (const uint32_t*)(cnt + cur), stp);
+                           (const uint32_t*)(cnt + 2 * cur), stp);
         hipError_t le = hipGetLastError();
         if (le != hipSuccess) return hip_status(c, le, "tail launch");
         launches += 1;
@@ -4229,11 +4294,11 @@ ear_status run_backward_batch(Ctx* c, uint32_t n_items, DeviceScene* const* scen
             if (batch)
                 k_generate<true><<<persistent_grid(c, n_chunk, waves), kBlock, 0, st>>>(
                     di, dsegs.as<GenSeg>(), dsegoff.as<uint32_t>(), (uint32_t)segs.size(), n_chunk,
-                    dplan.as<uint32_t>(), max_rec, 0u, q[0], cnt + 0, SQ, cnt + 2, stp);
+                    dplan.as<uint32_t>(), max_rec, 0u, 0u, q[0], cnt + 0, SQ, cnt + 2, stp);
             else
                 k_generate<false><<<persistent_grid(c, n_chunk, waves), kBlock, 0, st>>>(
                     di, dsegs.as<GenSeg>(), dsegoff.as<uint32_t>(), (uint32_t)segs.size(), n_chunk,
-                    dplan.as<uint32_t>(), max_rec, 0u, q[0], cnt + 0, SQ, cnt + 2, stp);
+                    dplan.as<uint32_t>(), max_rec, 0u, 0u, q[0], cnt + 0, SQ, cnt + 2, stp);
             if (!all_local || all_score) k_zero_f32<<<1024, 256, 0, st>>>(T[0].t, (size_t)cap * nm_max * 8);
             k_zero_f32<<<1024, 256, 0, st>>>(T[0].r, (size_t)cap * nm_max);
             EAR_HIP_TRY(c, hipMemcpyAsync(pinned, cnt, 12, hipMemcpyDeviceToHost, st));
