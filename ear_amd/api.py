@@ -69,7 +69,7 @@ class Context:
         graph_iters > 0 replays the bounce loop as a captured HIP graph;
         tail_rays: the last <= tail_rays live rays go to one launch that
         traces each to its end (default: every ray when no scene of the call
-        has more than 64 triangles, else the last 2^20; 1 turns it off);
+        has more than 64 triangles, else the last 2^21; 1 turns it off);
         splat: 1 direct 128-bit atomics per ramp point, 2 records binned by
         time tile and accumulated in LDS (same histograms); 0 the tiled one
         when the call's (row, tile) keys fit in 8192 and its queues hold at

@@ -320,7 +320,8 @@ __device__ __forceinline__ void stat_drops(unsigned long long* stats, const Drop
 // and claim in 64 bits a refill cost about 300 instructions).
 struct Claim {
     uint32_t n, next, end, seg, seg_len, n_seg, want, fails;
-    __device__ __forceinline__ Claim(uint32_t n_, uint32_t gtid, uint32_t threads, const Fetch& f) {
+    // own: entries a wave has of a short queue (64, or fewer to spread it out)
+    __device__ __forceinline__ Claim(uint32_t n_, uint32_t gtid, uint32_t threads, const Fetch& f, uint32_t own = 64u) {
         n = (uint32_t)__builtin_amdgcn_readfirstlane((int)n_);
         n_seg = f.n_seg;
         seg = (uint32_t)__builtin_amdgcn_readfirstlane((int)((gtid >> 6) % n_seg));
@@ -331,8 +332,8 @@ struct Claim {
         want = f.chunk ? f.chunk : (n / 256u >= threads / 64u ? 64u : 0u);
         if (n <= threads) {
             const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)((threadIdx.x >> 6) * gridDim.x + blockIdx.x));
-            next = min(wave * 64u, n);
-            end = min(next + 64u, n);
+            next = min(wave * own, n);
+            end = min(next + own, n);
             fails = n_seg;
         }
     }
@@ -1380,66 +1381,96 @@ __global__ void __launch_bounds__(kShadeBlock, 6) k_shade(const InstDev* __restr
 // whose time is then set by the latency of a few walks.  The same device
 // functions in the same order: every path, and so every histogram sum, is
 // the wavefront loop's.  A path ends by a miss, a non-normal intensity, the
-// cut-off or max_bounces, so every lane's loop ends.  Not used with the
-// sphere estimator, hit logging or counter instrumentation.
+// cut-off or max_bounces, so every lane's loop ends.  Not used with hit
+// logging or counter instrumentation.
+//
+// A wave's lanes go through one segment of their paths together: walk, shade,
+// connect, sample.  A lane whose path has ended takes the next ray before the
+// next segment (with the lanes of a wave on one ray each until the longest
+// path ended, and each lane drawing its own hemisphere candidates, the
+// 12-triangle box of 1M rays took 21.7 ms here against 14.5).  A queue
+// shorter than the grid is spread over all its waves, down to kTailMin rays
+// each: a segment then waits for the longest of fewer walks, and the chip has
+// the waves to spare.
+constexpr uint32_t kTailMin = 8;
 template <int BLOCK, int LDS, int WIDTH, bool BATCH>
-__global__ void __launch_bounds__(BLOCK) k_tail(const InstDev* __restrict__ inst, int* gstack, uint32_t gthreads,
-                                                Queue q, const uint32_t* __restrict__ n_q,
-                                                unsigned long long* __restrict__ stats) {
+__global__ void __launch_bounds__(BLOCK, 4) k_tail(const InstDev* __restrict__ inst, int* gstack, uint32_t gthreads,
+                                                Queue q, const uint32_t* __restrict__ n_q, uint32_t max_rec,
+                                                Fetch fetch, unsigned long long* __restrict__ stats) {
     __shared__ int lds[LDS * BLOCK];
+    __shared__ HemiLds hl[BLOCK / 64];
     const uint32_t n = *n_q;
     const uint32_t gtid = blockIdx.x * BLOCK + threadIdx.x;
+    const uint32_t lane = lane_id();
+    const uint32_t waves = gridDim.x * (BLOCK / 64);
     uint32_t n_seg = 0, nsh = 0, ncon = 0, nvis = 0, ntri = 0;
     Drops drops;
-    for (uint32_t i = gtid; i < n; i += gridDim.x * BLOCK) {
-        float4 ro = q.o[i], rd = q.d[i];
-        uint4 rm = q.m[i];
-        const uint32_t id = BATCH ? rm.w : 0;
+    Claim claim(n, gtid, gridDim.x * BLOCK, fetch, min(64u, max(kTailMin, n / waves + (n % waves ? 1u : 0u))));
+    bool live = false;
+    float4 ro{}, rd{};
+    uint4 rm{};
+    uint32_t id = 0;
+    for (;;) {
+        const uint64_t idle = __ballot(!live);
+        if (idle && !claim.exhausted()) {
+            const uint32_t mine = claim.take(fetch, idle, lane);
+            if (mine != 0xFFFFFFFFu) {
+                ro = q.o[mine];
+                rd = q.d[mine];
+                rm = q.m[mine];
+                id = BATCH ? rm.w : 0u;
+                live = true;
+            }
+        }
+        if (__ballot(live) == 0) break;
         const InstDev& In = inst[id];
         const RenderParams& P = In.P;
         const Traversal T = make_trav(In, gstack, gthreads);
         const int band = (int)(rm.z & 0xFFu);
-        for (;;) {
-            const uint32_t k = ((rm.z >> 8) & 0xFFFFu) + 1;  // this segment's bounce number
-            float bt_t = 1000000.0f;
-            int bs = -1;
-            uint32_t bo = 0;
-            traverse<LDS, BLOCK, WIDTH, false, false>(T, V3{ro.x, ro.y, ro.z}, V3{rd.x, rd.y, rd.z}, bt_t, bs, bo,
-                                                      lds + threadIdx.x, gtid, nvis, ntri);
-            ++n_seg;
-            if (bs < 0) break;  // no hit ends the path (src/Scene.cpp:166)
-            Rng rng;
-            V3 p, nrm, prev, d;
-            float I = 0.0f, L = 0.0f, spec = 0.0f, seg = 0.0f;
-            int bt = kReflect;
-            bool alive = false;
-            surface_hit(In, P, band, ro, rd, rm, make_int2(__float_as_int(bt_t), bs), rng, p, nrm, prev, d, I, L, spec,
-                        seg, bt, alive);
-            if (!alive) break;
-            for (uint32_t r = 0; r < P.n_rec; ++r) {
-                float c = 0.0f;
-                const RecParams& R = P.rec[r];
-                if (!nee_weight(P, R, band, p, nrm, prev, bt, spec, I, k, c)) continue;
-                // Scene::Connect: the segment from the hit point to the recorder
-                V3 dv = sub(V3{R.px, R.py, R.pz}, p);
-                float st = 0.0f;
-                int ss = -1;
-                uint32_t so = 0;
-                ++nsh;
-                const bool occ = traverse<LDS, BLOCK, WIDTH, true, false>(T, p, dv, st, ss, so, lds + threadIdx.x,
-                                                                          gtid, nvis, ntri);
-                if (!occ) {
-                    float l = length(dv);
-                    V3 lsdir = normalized(dv);
-                    record(make_hist(In), band, R, lsdir, c, (L + l) / 343.0f, L + l, drops);
-                    ++ncon;
-                }
+        const uint32_t k = ((rm.z >> 8) & 0xFFFFu) + 1;  // this segment's bounce number
+        int2 h = make_int2(0, -1);
+        {
+            Walker<LDS, BLOCK, WIDTH, false, false> w(lds + threadIdx.x, gstack, gtid, gthreads);
+            if (live) w.start(T, V3{ro.x, ro.y, ro.z}, V3{rd.x, rd.y, rd.z}, 1000000.0f);
+            while (__ballot(!w.idle())) w.step(T, nvis, ntri);
+            h = make_int2(__float_as_int(w.best_t), w.best_s);
+        }
+        n_seg += live ? 1u : 0u;
+        Rng rng;
+        V3 p{0, 0, 0}, nrm{0, 0, 0}, prev{0, 0, 0}, d{0, 0, 0};
+        float I = 0.0f, L = 0.0f, spec = 0.0f;
+        float seg = __int_as_float(0x7f800000);  // segment length; +inf for a miss
+        int bt = kReflect;
+        bool alive = false;
+        // no hit ends the path (src/Scene.cpp:166)
+        if (live && h.y >= 0) surface_hit(In, P, band, ro, rd, rm, h, rng, p, nrm, prev, d, I, L, spec, seg, bt, alive);
+        const bool nee = P.estimator == EAR_EST_NEE;
+        if (live && !nee)
+            ncon += sphere_deposits(make_hist(In), P, band, V3{ro.x, ro.y, ro.z}, normalized(V3{rd.x, rd.y, rd.z}), seg,
+                                    ro.w, rd.w, k - 1, drops);
+        for (uint32_t r = 0; r < max_rec; ++r) {
+            float c = 0.0f;
+            const RecParams& R = P.rec[r];
+            const bool emit = alive && nee && r < P.n_rec && nee_weight(P, R, band, p, nrm, prev, bt, spec, I, k, c);
+            // Scene::Connect: the segment from the hit point to the recorder
+            const V3 dv = sub(V3{R.px, R.py, R.pz}, p);
+            Walker<LDS, BLOCK, WIDTH, true, false> w(lds + threadIdx.x, gstack, gtid, gthreads);
+            if (emit) w.start(T, p, dv, 0.0f);
+            while (__ballot(!w.idle())) w.step(T, nvis, ntri);
+            nsh += emit ? 1u : 0u;
+            if (emit && !w.found()) {
+                const float l = length(dv);
+                record(make_hist(In), band, R, normalized(dv), c, (L + l) / 343.0f, L + l, drops);
+                ++ncon;
             }
-            if ((double)I < P.cutoff || k >= P.max_bounces) break;
+        }
+        live = alive && !((double)I < P.cutoff) && k < P.max_bounces;
+        const V3 hv = sample_hemi_wave(live, true, rng, nrm, hl[threadIdx.x >> 6]);
+        if (live) {
             // REFRACT: the negated normal and the incoming direction; REFLECT:
             // the mirror direction about the ray-facing normal (src/Scene.cpp:65-74)
-            V3 rdir = bt == kRefract ? d : reflect(d, nrm);
-            V3 v = sample_hemi_spec(rng, nrm, rdir, spec);
+            const V3 rdir = bt == kRefract ? d : reflect(d, nrm);
+            const V3 v = blend_spec(hv, rdir, spec);
             ro = make_float4(p.x, p.y, p.z, I);
             rd = make_float4(v.x, v.y, v.z, L);
             rm = make_uint4(rm.x, rng.draw, (uint32_t)band | (k << 8), id);
@@ -2261,7 +2292,7 @@ void pick_b(const TravCfg& c, ExtendFn* e, ShadowFn* s) {
     }
 }
 
-using TailFn = void (*)(const InstDev*, int*, uint32_t, Queue, const uint32_t*, unsigned long long*);
+using TailFn = void (*)(const InstDev*, int*, uint32_t, Queue, const uint32_t*, uint32_t, Fetch, unsigned long long*);
 
 template <int B, int L>
 TailFn tail_for(int width, bool batch) {
@@ -2964,22 +2995,27 @@ ear_status run_batch(Ctx* c, uint32_t n_items, DeviceScene* const* scenes, const
     };
     // the tail: every ray emitted and few live ones left (queue cur, of
     // pinned[2 cur] rays, read by finished); one launch traces them to their ends
-    // (tail_rays 0: 2^20 live rays, measured best on the 200k-triangle hall,
-    // or every ray when no scene has more than 64 triangles: their walks are
-    // so short that the queues between the wavefront kernels cost more than
-    // the phase divergence of one launch (12-triangle box, 3M rays: 3.25e9
-    // against 2.11e9 segments/s); 1: no tail launch)
+    // (tail_rays 0: 2^21 live rays, or every ray when no scene has more than
+    // 64 triangles: their walks are so short that the queues between the
+    // wavefront kernels cost more than a segment's wait for the wave's longest
+    // walk.  The 12-triangle box of 1M rays: 22 ms, 41 with the last 2^20 only;
+    // 32 rooms at 2^20, 2^21, 2^22, all: 116, 113, 110, 100 ms; the 200k hall
+    // 326, 321, 319, 356; 12 keyframes of the 100k hall 72.3, 72.2, 74.0,
+    // 86.7: rooms would take more, halls do not, and their trees do not tell
+    // them apart; 1: no tail launch)
     uint32_t max_tris = 0;
     for (uint32_t i = 0; i < n_items; ++i) max_tris = std::max(max_tris, inst[i].n_tris);
-    const uint32_t tail_default = max_tris <= 64 ? 0xFFFFFFFFu : (1u << 20);
+    const uint32_t tail_default = max_tris <= 64 ? 0xFFFFFFFFu : (1u << 21);
     const uint32_t tail_rays = tu.tail_rays == 0 ? tail_default : (tu.tail_rays == 1 ? 0u : tu.tail_rays);
-    bool tail_ok = tail_rays > 0 && !instr && !any_log;
-    for (uint32_t i = 0; i < n_items; ++i) tail_ok = tail_ok && inst[i].P.estimator == EAR_EST_NEE;
+    const bool tail_ok = tail_rays > 0 && !instr && !any_log;
     const TailFn ft = tail_ok ? pick_tail(cfg_e) : nullptr;
     auto tail = [&](int cur, bool* done) -> ear_status {
         if (*done || !ft || pinned[4] != total32 || pinned[2 * cur] > tail_rays) return EAR_OK;
-        hipLaunchKernelGGL(ft, dim3(g_ext), dim3(cfg_e.block), 0, st, di, gsp, gthreads, qq[cur],
-                           (const uint32_t*)(cnt + 2 * cur), stp);
+        // (one round of resident blocks: the waves of a second one would start
+        // on the last rays when the first ends)
+        const uint32_t g_tail = std::min(cap_e, cap_for((const void*)ft, cfg_e.block));
+        hipLaunchKernelGGL(ft, dim3(g_tail), dim3(cfg_e.block), 0, st, di, gsp, gthreads, qq[cur],
+                           (const uint32_t*)(cnt + 2 * cur), (uint32_t)max_recs, fq_e, stp);
         hipError_t le = hipGetLastError();
         if (le != hipSuccess) return hip_status(c, le, "tail launch");
         launches += 1;

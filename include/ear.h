@@ -382,7 +382,7 @@ typedef struct {
                                 (1..64, default 16) */
     uint32_t tail_rays;      /* once every ray is emitted and at most this many are live,
                                 one launch traces each through all its remaining segments
-                                (same histograms); 0: default, 2^20, or every ray when no
+                                (same histograms); 0: default, 2^21, or every ray when no
                                 scene has more than 64 triangles; 1: never (the bounce loop
                                 to the end) */
     uint32_t splat;          /* EAR_SPLAT_*: how the shadow kernels add ramps to the
