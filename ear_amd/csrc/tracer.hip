@@ -2931,8 +2931,8 @@ ear_status run_batch(Ctx* c, uint32_t n_items, DeviceScene* const* scenes, const
     const uint32_t nseg = tu.fetch_segments ? std::min<uint32_t>(tu.fetch_segments, kMaxSeg) : kSegDefault;
     const Fetch fq_e{segc.as<uint32_t>(), refill, fchunk, nseg},
         fq_s{segc.as<uint32_t>() + kMaxSeg * kSegStride, refill, fchunk, nseg};
-    // one iteration; cur = the queue it consumes
-    auto iteration = [&](int cur) {
+    // tops queue cur up with new rays
+    auto generate = [&](int cur) {
         // [2 q] rays of queue q, [2 q + 1] the shadow requests made with it as
         // the output queue; [4] generation cursor, [6..8] plan
         uint32_t *nq = cnt + 2 * cur, *nsq = cnt + 2 * (1 - cur) + 1;
@@ -2945,21 +2945,10 @@ ear_status run_batch(Ctx* c, uint32_t n_items, DeviceScene* const* scenes, const
             k_generate<false><<<g_gen, kBlock, 0, st>>>(di, dsegs.as<GenSeg>(), dsegoff.as<uint32_t>(), n_segs, 0u,
                                                         cnt + 6, (uint32_t)max_recs, any_mesh, dense, qq[cur], nq, SQ,
                                                         nsq, stp);
-        EventPair* e1 = timed ? &mk(ev_ext) : nullptr;
-        if (e1) hipEventRecord(e1->a, st);
-        hipLaunchKernelGGL(fe, dim3(g_ext), dim3(cfg_e.block), 0, st, di, gsp, gthreads, qq[cur], (const uint32_t*)nq,
-                           hits.as<int2>(), stp, fq_e);
-        if (e1) hipEventRecord(e1->b, st);
-        EventPair* e2 = timed ? &mk(ev_sha) : nullptr;
-        if (e2) hipEventRecord(e2->a, st);
-        unsigned long long* n_out = (unsigned long long*)(cnt + 2 * (1 - cur));
-        if (batch)
-            k_shade<true><<<g_shade, kShadeBlock, 0, st>>>(di, qq[cur], nq, hits.as<int2>(), qq[1 - cur], SQ, n_out,
-                                                           (uint32_t)max_recs, stp);
-        else
-            k_shade<false><<<g_shade, kShadeBlock, 0, st>>>(di, qq[cur], nq, hits.as<int2>(), qq[1 - cur], SQ, n_out,
-                                                            (uint32_t)max_recs, stp);
-        if (e2) hipEventRecord(e2->b, st);
+    };
+    // traces the shadow requests of the iteration that consumes queue cur
+    auto connect = [&](int cur) {
+        uint32_t* nsq = cnt + 2 * (1 - cur) + 1;
         EventPair* e3 = timed ? &mk(ev_shw) : nullptr;
         if (e3) hipEventRecord(e3->a, st);
         hipLaunchKernelGGL(fs, dim3(g_shw), dim3(cfg_s.block), 0, st, di, gsp, gthreads, SQ, (const uint32_t*)nsq,
@@ -2981,6 +2970,27 @@ ear_status run_batch(Ctx* c, uint32_t n_items, DeviceScene* const* scenes, const
             if (e4) hipEventRecord(e4->b, st);
             launches += 4;
         }
+    };
+    // one iteration; cur = the queue it consumes
+    auto iteration = [&](int cur) {
+        uint32_t* nq = cnt + 2 * cur;
+        generate(cur);
+        EventPair* e1 = timed ? &mk(ev_ext) : nullptr;
+        if (e1) hipEventRecord(e1->a, st);
+        hipLaunchKernelGGL(fe, dim3(g_ext), dim3(cfg_e.block), 0, st, di, gsp, gthreads, qq[cur], (const uint32_t*)nq,
+                           hits.as<int2>(), stp, fq_e);
+        if (e1) hipEventRecord(e1->b, st);
+        EventPair* e2 = timed ? &mk(ev_sha) : nullptr;
+        if (e2) hipEventRecord(e2->a, st);
+        unsigned long long* n_out = (unsigned long long*)(cnt + 2 * (1 - cur));
+        if (batch)
+            k_shade<true><<<g_shade, kShadeBlock, 0, st>>>(di, qq[cur], nq, hits.as<int2>(), qq[1 - cur], SQ, n_out,
+                                                           (uint32_t)max_recs, stp);
+        else
+            k_shade<false><<<g_shade, kShadeBlock, 0, st>>>(di, qq[cur], nq, hits.as<int2>(), qq[1 - cur], SQ, n_out,
+                                                            (uint32_t)max_recs, stp);
+        if (e2) hipEventRecord(e2->b, st);
+        connect(cur);
         // the consumed queue, the shadow queue and the fetch counters
         k_reset_iter<<<1, 64, 0, st>>>(cnt, (1u << (2 * cur)) | (1u << (2 * (1 - cur) + 1)), segc.as<uint32_t>(), 2 * kMaxSeg);
         launches += 6;
@@ -3025,7 +3035,21 @@ ear_status run_batch(Ctx* c, uint32_t n_items, DeviceScene* const* scenes, const
     const uint32_t max_iters = max_bounces + 2 + (uint32_t)((total_rays + cap_rays - 1) / cap_rays) * (max_bounces + 1);
     int cur = 0;
     bool done = false;
-    if (eager) {
+    if (ft && dense && total32 <= cap_rays && total32 <= tail_rays) {
+        // all rays are the tail's from the first segment: emission, the
+        // connections that an emitting mesh makes, one launch.  (Of the four
+        // bounce iterations before a look at the counts, each with the whole
+        // population's first hits on the same few bins, the 1M-ray box spent
+        // 4 of its 22 ms and a room with an emitting mesh 5 of 36.)
+        generate(0);
+        if (any_mesh) connect(0);
+        k_reset_iter<<<1, 64, 0, st>>>(cnt, 8u, segc.as<uint32_t>(), 2 * kMaxSeg);
+        launches += 4;
+        pinned[0] = pinned[4] = total32;
+        status = tail(0, &done);
+    }
+    if (done || status != EAR_OK) {
+    } else if (eager) {
         const uint32_t every = 4;
         while (!done && status == EAR_OK) {
             for (uint32_t k = 0; k < every; ++k) {
