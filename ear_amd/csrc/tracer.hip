@@ -118,31 +118,6 @@ __device__ __forceinline__ uint32_t wave_append(uint32_t* counter, bool pred) {
     return base + (uint32_t)__popcll(below);
 }
 
-// Block-wide append: like wave_append with one atomic per block instead of
-// per wave (a queue counter is one address; per-wave atomics from every wave
-// of the GPU serialise there).  Every thread of the block must call it;
-// `sc` is block-shared scratch of BLOCK / 64 + 1 words that consecutive calls
-// must not share (the caller alternates two).
-template <int BLOCK>
-__device__ __forceinline__ uint32_t block_append(uint32_t* counter, bool pred, uint32_t* sc) {
-    constexpr uint32_t kWaves = BLOCK / 64;
-    const uint32_t lane = lane_id(), wave = threadIdx.x >> 6;
-    const uint64_t mask = __ballot(pred);
-    if (lane == 0) sc[wave] = (uint32_t)__popcll(mask);
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        uint32_t tot = 0;
-        for (uint32_t w = 0; w < kWaves; ++w) {
-            const uint32_t cw = sc[w];
-            sc[w] = tot;
-            tot += cw;
-        }
-        sc[kWaves] = tot ? atomicAdd(counter, tot) : 0u;
-    }
-    __syncthreads();
-    return sc[kWaves] + sc[wave] + (uint32_t)__popcll(mask & ((1ull << lane) - 1ull));
-}
-
 // Two appends of a block with one atomic: a wave's `a` entries to the counter
 // in the low word and `b` to the one in the high word of `counter` (neither
 // overflows: a queue holds fewer than 2^32).  Adds to one address take about
@@ -3289,7 +3264,6 @@ struct Tangents {
         return t[((size_t)q * 8 + field) * cap + slot];
     }
     __device__ float& refl(uint32_t q, uint32_t slot) const { return r[(size_t)q * cap + slot]; }
-    __device__ float& row(uint32_t j, uint32_t slot) const { return t[(size_t)j * cap + slot]; }  // score form
 };
 
 // The adjoint histograms as prefix sums: row (band, channel) holds bins + 1
@@ -3356,7 +3330,9 @@ __device__ double ramp_adjoint(const double2* pre, uint32_t nb, int s, int w, do
     const int lo = s < 0 ? 0 : s;
     const int hi = s + w > (int)nb ? (int)nb : s + w;
     if (lo >= hi) return 0.0;
-    const double2 a = pre[lo], b = pre[hi];
+    typedef double f64x2 __attribute__((ext_vector_type(2)));
+    const f64x2 a = *(const __attribute__((address_space(1))) f64x2*)(pre + lo),
+                b = *(const __attribute__((address_space(1))) f64x2*)(pre + hi);
     return ((double)(w + s) * (b.x - a.x) - (b.y - a.y)) / (double)w * per_c;
 }
 
@@ -3573,7 +3549,7 @@ __global__ void __launch_bounds__(kBlock) k_shade_ad(const InstDev* __restrict__
                     cont = !((double)I < P.cutoff) && k < P.max_bounces;
                 }
                 if (cont) {
-                    // hemisphere sample and blend exactly as sample_hemi_spec
+                    // hemisphere sample and blend exactly as k_shade does
                     V3 hs = sample_hemi(rng, nrm);
                     V3 rdir = bt == kRefract ? d : reflect(d, nrm);
                     float gg = 1.0f - spec;
@@ -3656,148 +3632,162 @@ __global__ void __launch_bounds__(kBlock) k_shade_ad(const InstDev* __restrict__
     block_grad_flush(A0, band_acc, g_refl, g_spec, &red[0][0]);
 }
 
-// Connection requests of the local adjoint: the hit point, the gradient
-// weights the connection adds when it is visible, and which recorder,
-// band, material and instance it belongs to.
-struct AdjShadowQ {
-    float4* p;  // {px, py, pz, -}
-    uint4* m;   // {rec | band << 8 | mat << 16, instance, -, -}
-    float4* w;  // [4 per request]: d/drefl_q (q = 0..7), then d/dspec_q (q = 0..7), each times dL/dc
-};
-
-// The score form (EAR_FLAG_ADJ_SCORE): a queue entry whose metadata carries
-// kContFlag is a continuation path.  Its tangent rows hold S (the weight of
-// its spawning material, zero elsewhere) and, in row n_mat, the vertex that
-// spawned it (its stream's key).
-constexpr uint32_t kContFlag = 1u << 31;
-// a vertex spawns a continuation with probability min(1, kScoreRate F), F
-// its rim flux (the rim term's weight: the least variance for a given
-// number of continuations)
+// a vertex of the score form spawns a continuation with probability
+// min(1, kScoreRate F), F its rim flux (the rim term's weight: the least
+// variance for a given number of continuations)
 constexpr float kScoreRate = 0.05f;
+constexpr int kAdjLds = 8;  // k_adj_paths' LDS entries of a traversal stack
 
-struct ContOut {  // where a score-form vertex appends its continuation
-    Queue q;
-    uint32_t* n;
-    Tangents t;
-};
+__device__ __forceinline__ void add_grad(double* p, double v) {
+    if (v != 0.0) __hip_atomic_fetch_add((__attribute__((address_space(1))) double*)p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
 
 // The adjoint with EAR_FLAG_ADJ_LOCAL (or EAR_FLAG_ADJ_SCORE) for every ray:
 // no direction or position tangents travel between vertices, so a ray
 // carries only dlogI/drefl (n_mat floats) and, in the score form, S (n_mat
-// floats).  At each connection of a hit on material m,
+// floats).  At each visible connection of a hit on material m,
 // d c / d spec_m = sign I air^l 2 / (4 pi l^2) (lobe - diffuse) and
-// d c / d refl_q = c dlogI/drefl_q; the score form adds c S_q to d c / dspec_q.
-// Times dL/dc they are queued as a request whose visibility k_adj_vis
-// decides, as k_shade queues the forward's.  Same primal and draws as
-// k_shade; arrays are indexed at compile time only.
+// d c / d refl_q = c dlogI/drefl_q; the score form adds c S_q to d c / dspec_q;
+// times dL/dc they join the lane's sums, which go to the gradient of their
+// instance and band when the lane moves to another or ends.  Same primal and
+// draws as k_shade; the sums are indexed at compile time only.
 //
 // SCORE: after its connections, a vertex whose path goes on adds to S_m
 // (m its material) d log p(v)/ds - F for the direction v it drew, and with
-// probability q = min(1, kScoreRate F) appends a continuation leaving the
-// vertex along a rim direction (score_rim_dir) with weight -F / q on spec_m,
-// adding F / q to S_m.  A continuation replays transport only:
-// no refl tangents, no explicit lobe term, no score, no spawns.
-// CONT: every entry of the queue is a continuation (the continuations' own
-// queues), so the main paths' steps compile away.
-template <bool BATCH, bool SCORE, bool CONT = false>
-__global__ void __launch_bounds__(kBlock) k_shade_adl(const InstDev* __restrict__ inst, Queue qin,
-                                                       const uint32_t* __restrict__ n_in,
-                                                       const int2* __restrict__ hits, Tangents tin, Queue qout,
-                                                       uint32_t* __restrict__ n_out, Tangents tout, AdjShadowQ aq,
-                                                       uint32_t* __restrict__ n_aq, uint32_t max_rec, AdjArgs A0,
-                                                       const AdjArgs* __restrict__ adj, ContOut co,
-                                                       unsigned long long* __restrict__ stats) {
-    __shared__ uint32_t sc[6][kBlock / 64 + 1];  // scratch of the block-wide appends, alternated
+// probability q = min(1, kScoreRate F) a continuation leaves the vertex along
+// a rim direction (score_rim_dir) with weight -F / q on spec_m, F / q being
+// added to S_m.  A continuation replays transport only: no refl tangents, no
+// explicit lobe term, no score, no spawns.  The lane follows it to its end at
+// once and then takes its main path up again, so it needs no queue.
+//
+// One launch carries the rays of every band to their ends, as k_tail does (a
+// wave's lanes go through one segment together and refill).  A bounce at a
+// time through queues, with a request of 16 weights per connection, a pair of
+// tangent arrays and the continuations' own queues, launches of some 100 us
+// each for a few rays and each band by itself made the 1M-ray box 129 ms and 8
+// rooms 117 ms; here 69 and 77.  Bound by the vector units at the occupancy
+// that the registers allow: with every array in registers (206 to 225 of
+// them, two waves a SIMD) the box took 86, so the path's two arrays, indexed
+// by material anyway, and a waiting main path are in LDS, which half the usual
+// stack makes room for (168 registers, three waves; four waves spill: 100).
+template <int WIDTH, bool BATCH, bool SCORE>
+__global__ void __launch_bounds__(kBlock, 3) k_adj_paths(const InstDev* __restrict__ inst, int* gstack,
+                                                         uint32_t gthreads, Queue q, const uint32_t* __restrict__ n_q,
+                                                         uint32_t max_rec, AdjArgs A0,
+                                                         const AdjArgs* __restrict__ adj, Fetch fetch) {
+    constexpr int LDS = kAdjLds;
+    __shared__ int lds[LDS * kBlock];
     __shared__ HemiLds hl[kBlock / 64];
-    const uint32_t n = *n_in;
-    uint32_t n_done = 0;
-    for (uint32_t base = blockIdx.x * kBlock; base < n; base += gridDim.x * kBlock) {
-        const uint32_t i = base + threadIdx.x;
-        const uint32_t parity = (base / (gridDim.x * kBlock)) & 1u;
-        bool cont = false, alive = false, contn = false, spawn = false;
-        Rng rng;
-        float4 no{}, nd{};
-        uint4 nmeta{};
-        float drefl[kAdMaxMat], sacc[kAdMaxMat];
+    __shared__ float4 mo[kBlock], md[kBlock];  // a continuation's main path
+    __shared__ uint4 mm[kBlock];
+    const uint32_t n = *n_q;
+    const uint32_t gtid = blockIdx.x * kBlock + threadIdx.x;
+    const uint32_t lane = lane_id();
+    const uint32_t waves = gridDim.x * (kBlock / 64);
+    uint32_t nvis = 0, ntri = 0;
+    Claim claim(n, gtid, gridDim.x * kBlock, fetch, min(64u, max(kTailMin, n / waves + (n % waves ? 1u : 0u))));
+    double g_refl[kAdMaxMat], g_spec[kAdMaxMat];
+    __shared__ float drefl_s[kAdMaxMat * kBlock], sacc_s[kAdMaxMat * kBlock];
+    float* drefl = drefl_s + threadIdx.x;
+    float* sacc = sacc_s + threadIdx.x;
 #pragma unroll
-        for (int q = 0; q < kAdMaxMat; ++q) drefl[q] = sacc[q] = 0.0f;
-        uint32_t nm = A0.n_mat, id = 0, k = 0, mat = 0, n_rec = 0, kspawn = 0, sdraw = 0, ray = 0;
-        int band = 0, bt = kReflect;
-        float I = 0.0f, L = 0.0f, spec = 0.0f, wcont = 0.0f;
-        V3 p{0, 0, 0}, nrm{0, 0, 0}, prev{0, 0, 0}, vdir{0, 0, 0}, rdir{0, 0, 0}, vb{0, 0, 0};
-        if (i < n) {
-            const float4 ro = qin.o[i];
-            const float4 rd = qin.d[i];
-            const uint4 rm = qin.m[i];
-            id = BATCH ? rm.w : 0u;
-            ray = rm.x;
-            const InstDev& In = inst[id];
-            const RenderParams& P = In.P;
-            nm = (BATCH ? adj[id] : A0).n_mat;
-            n_rec = P.n_rec;
-            band = (int)(rm.z & 0xFFu);
-            k = ((rm.z >> 8) & 0xFFFFu) + 1;
-            contn = CONT || (SCORE && (rm.z & kContFlag) != 0u);
-            const int2 h = hits[i];
-            if (h.y >= 0) {
-                const float t = __int_as_float(h.x);
-                const V3 o{ro.x, ro.y, ro.z};
-                const V3 d{rd.x, rd.y, rd.z};
-                p = V3{o.x + d.x * t, o.y + d.y * t, o.z + d.z * t};
-                const float4 nmv = ldg(In.nm + h.y);
-                const V3 N{nmv.x, nmv.y, nmv.z};
-                nrm = dot(N, d) > 0.0f ? V3{N.x * -1.0f, N.y * -1.0f, N.z * -1.0f} : N;
-                mat = __float_as_uint(nmv.w);
-                const float4 mb = ldg(In.mat_band + 3 * mat + band);
-                if (contn) {
-                    kspawn = __float_as_uint(tin.row(nm, i));
-                    score_rng_init(rng, P.seed, rm.x, P.ctx_word[band], P.instance, kspawn, rm.y);
-                } else {
-                    rng.init(P.seed, rm.x, P.ctx_word[band], P.instance, rm.y);
-                }
-                if (mb.x >= 0.0f) bt = (rng.next() <= mb.x) ? kReflect : kRefract;
-                spec = mb.y;
-                if (bt == kRefract) nrm = neg(nrm);
-                const float l = length(sub(p, o));
-                I = ro.w;
-                I *= powf_ear_l2(P.air[band], P.l2_air[band], l);
-                L = rd.w + l;
-                I *= mb.z;
-                prev = normalized(d);
+    for (int m = 0; m < kAdMaxMat; ++m) {
+        g_refl[m] = g_spec[m] = 0.0;
+        drefl[m * kBlock] = sacc[m * kBlock] = 0.0f;
+    }
+    uint32_t key = 0xFFFFFFFFu;  // instance and band of the sums
+    int kband = 0;
+    bool live = false, contn = false;  // on a path; on a continuation
+    float4 ro{}, rd{};                 // the path's state
+    uint4 rm{};
+    uint32_t id = 0, cmat = 0, kspawn = 0;  // a continuation's material and vertex
+    float wcont = 0.0f;                     // and weight
+    for (;;) {
+        const uint64_t idle = __ballot(!live);
+        if (idle && !claim.exhausted()) {
+            const uint32_t mine = claim.take(fetch, idle, lane);
+            if (mine != 0xFFFFFFFFu) {
+                ro = q.o[mine];
+                rd = q.d[mine];
+                rm = q.m[mine];
+                id = BATCH ? rm.w : 0u;
+                const int b = (int)(rm.z & 0xFFu);
+                if (key != 0xFFFFFFFFu && (key != id || kband != b)) {
+                    const AdjArgs& A = BATCH ? adj[key] : A0;
+                    double* gk = A.grad_copy() + (size_t)kband * 2 * A.n_mat;
 #pragma unroll
-                for (int q = 0; q < kAdMaxMat; ++q) {
-                    if ((uint32_t)q < nm) {
-                        drefl[q] = contn ? 0.0f : tin.refl(q, i) + ((uint32_t)q == mat ? 1.0f / mb.z : 0.0f);
-                        if (SCORE) sacc[q] = tin.row(q, i);
+                    for (int m = 0; m < kAdMaxMat; ++m) {
+                        if ((uint32_t)m < A.n_mat) {
+                            add_grad(gk + m, g_refl[m]);
+                            add_grad(gk + A.n_mat + m, g_spec[m]);
+                        }
+                        g_refl[m] = g_spec[m] = 0.0;
                     }
                 }
-                alive = is_normal(I);
-                if (alive) {
-                    cont = !((double)I < P.cutoff) && k < P.max_bounces;
-                    if (cont) rdir = bt == kRefract ? d : reflect(d, nrm);
-                }
+                key = id;
+                kband = b;
+#pragma unroll
+                for (int m = 0; m < kAdMaxMat; ++m) drefl[m * kBlock] = sacc[m * kBlock] = 0.0f;
+                live = true;
+                contn = false;
             }
         }
+        if (__ballot(live) == 0) break;
+        const InstDev& In = inst[id];
+        const RenderParams& P = In.P;
+        const AdjArgs& A = BATCH ? adj[id] : A0;
+        const Traversal T = make_trav(In, gstack, gthreads);
+        const int band = (int)(rm.z & 0xFFu);
+        const uint32_t k = ((rm.z >> 8) & 0xFFFFu) + 1;
+        int2 h = make_int2(0, -1);
         {
-            const V3 hv = sample_hemi_wave(cont, true, rng, nrm, hl[threadIdx.x >> 6]);
-            if (cont) {
-                vdir = blend_spec(hv, rdir, spec);
-                no = make_float4(p.x, p.y, p.z, I);
-                nd = make_float4(vdir.x, vdir.y, vdir.z, L);
-                nmeta = make_uint4(ray, rng.draw, (uint32_t)band | (k << 8) | (contn ? kContFlag : 0u), id);
-            }
+            Walker<LDS, kBlock, WIDTH, false, false> w(lds + threadIdx.x, gstack, gtid, gthreads);
+            if (live) w.start(T, V3{ro.x, ro.y, ro.z}, V3{rd.x, rd.y, rd.z}, 1000000.0f);
+            while (__ballot(!w.idle())) w.step(T, nvis, ntri);
+            h = make_int2(__float_as_int(w.best_t), w.best_s);
         }
-        // connections to every recorder (src/Scene.cpp:185-268), queued with
-        // their gradient weights
+        Rng rng;
+        V3 p{0, 0, 0}, nrm{0, 0, 0};
+        float I = 0.0f, L = 0.0f, spec = 0.0f;
+        uint32_t mat = 0;
+        int bt = kReflect;
+        bool alive = false, cont = false;
+        if (live && h.y >= 0) {
+            const float t = __int_as_float(h.x);
+            const V3 o{ro.x, ro.y, ro.z};
+            const V3 d{rd.x, rd.y, rd.z};
+            p = V3{o.x + d.x * t, o.y + d.y * t, o.z + d.z * t};
+            const float4 nmv = ldg(In.nm + h.y);
+            const V3 N{nmv.x, nmv.y, nmv.z};
+            nrm = dot(N, d) > 0.0f ? V3{N.x * -1.0f, N.y * -1.0f, N.z * -1.0f} : N;
+            mat = __float_as_uint(nmv.w);
+            const float4 mb = ldg(In.mat_band + 3 * mat + band);
+            if (SCORE && contn)
+                score_rng_init(rng, P.seed, rm.x, P.ctx_word[band], P.instance, kspawn, rm.y);
+            else
+                rng.init(P.seed, rm.x, P.ctx_word[band], P.instance, rm.y);
+            if (mb.x >= 0.0f) bt = (rng.next() <= mb.x) ? kReflect : kRefract;
+            spec = mb.y;
+            if (bt == kRefract) nrm = neg(nrm);
+            const float l = length(sub(p, o));
+            I = ro.w;
+            I *= powf_ear_l2(P.air[band], P.l2_air[band], l);
+            L = rd.w + l;
+            I *= mb.z;
+            if (!contn) drefl[mat * kBlock] += 1.0f / mb.z;
+            alive = is_normal(I);
+            if (alive) cont = !((double)I < P.cutoff) && k < P.max_bounces;
+        }
+        // connections to every recorder (src/Scene.cpp:185-268), then the
+        // segment to it (Scene::Connect, src/Scene.cpp:84-96)
         for (uint32_t r = 0; r < max_rec; ++r) {
+            const RecParams& R = P.rec[r];
+            const V3 dv = sub(V3{R.px, R.py, R.pz}, p);
             bool emit = false;
             float ds = 0.0f, ac = 0.0f;
-            if (alive && r < n_rec) {
-                const RenderParams& P = inst[id].P;
-                const AdjArgs& A = BATCH ? adj[id] : A0;
-                const RecParams& R = P.rec[r];
-                const V3 dv = sub(V3{R.px, R.py, R.pz}, p);
+            if (alive && r < P.n_rec) {
                 const V3 lsdir = normalized(dv);
+                const V3 prev = normalized(V3{rd.x, rd.y, rd.z});
                 if (dot(lsdir, nrm) > 0.0f) {
                     float diff, sf;
                     if (bt == kReflect) {
@@ -3819,193 +3809,102 @@ __global__ void __launch_bounds__(kBlock) k_shade_adl(const InstDev* __restrict_
                     c *= geo_inv;
                     if (is_normal(c)) {
                         if (k & 1u) c *= -1.0f;
-                        const double a_c =
-                            contribution_adjoint(P, A, band, R, lsdir, c, (L + ls) / 343.0f, L + ls);
+                        const double a_c = contribution_adjoint(P, A, band, R, lsdir, c, (L + ls) / 343.0f, L + ls);
                         if (a_c != 0.0) {
                             const double cnof =
                                 ((k & 1u) ? -1.0 : 1.0) * (double)I * (double)geo_air * (double)geo_inv;
-                            ds = contn ? 0.0f : (float)(a_c * cnof * ((double)kExpInt * (double)pw - (double)diff));
+                            ds = (float)(a_c * cnof * ((double)kExpInt * (double)pw - (double)diff));
                             ac = (float)(a_c * (double)c);
                             emit = true;
                         }
                     }
                 }
             }
-            const uint32_t slot = block_append<kBlock>(n_aq, emit, sc[r & 1u]);
-            if (emit) {
-                float ws[kAdMaxMat];
+            Walker<LDS, kBlock, WIDTH, true, false> w(lds + threadIdx.x, gstack, gtid, gthreads);
+            if (emit) w.start(T, p, dv, 0.0f);
+            while (__ballot(!w.idle())) w.step(T, nvis, ntri);
+            if (emit && !w.found()) {
+                if (!contn) {
 #pragma unroll
-                for (int q = 0; q < kAdMaxMat; ++q) ws[q] = ac * sacc[q] + ((uint32_t)q == mat ? ds : 0.0f);
-                aq.p[slot] = make_float4(p.x, p.y, p.z, 0.0f);
-                aq.m[slot] = make_uint4(r | ((uint32_t)band << 8) | (mat << 16), id, 0u, 0u);
-                aq.w[4 * (size_t)slot] = make_float4(ac * drefl[0], ac * drefl[1], ac * drefl[2], ac * drefl[3]);
-                aq.w[4 * (size_t)slot + 1] =
-                    make_float4(ac * drefl[4], ac * drefl[5], ac * drefl[6], ac * drefl[7]);
-                aq.w[4 * (size_t)slot + 2] = make_float4(ws[0], ws[1], ws[2], ws[3]);
-                aq.w[4 * (size_t)slot + 3] = make_float4(ws[4], ws[5], ws[6], ws[7]);
+                    for (int m = 0; m < kAdMaxMat; ++m) {
+                        g_refl[m] += (double)(ac * drefl[m * kBlock]);
+                        g_spec[m] += (double)(ac * sacc[m * kBlock] + ((uint32_t)m == mat ? ds : 0.0f));
+                    }
+                } else {
+                    const double v = (double)(ac * wcont);
+#pragma unroll
+                    for (int m = 0; m < kAdMaxMat; ++m)
+                        if ((uint32_t)m == cmat) g_spec[m] += v;
+                }
             }
         }
-        if (SCORE && !CONT && cont && !contn) {
-            // the direction just drawn leaves this vertex: its score, the rim
-            // flux and perhaps a continuation (after this vertex's connections,
-            // which that direction does not reach)
-            const RenderParams& P = inst[id].P;
-            const double cdir = (double)vdir.x * (double)rdir.x + (double)vdir.y * (double)rdir.y +
-                                (double)vdir.z * (double)rdir.z;
-            const double cr = (double)rdir.x * (double)nrm.x + (double)rdir.y * (double)nrm.y +
-                              (double)rdir.z * (double)nrm.z;
-            const double F = score_flux(cr, (double)spec);
-            double coef = score_dlogp(cdir, (double)spec) - F;
-            Rng rs;
-            score_rng_init(rs, P.seed, ray, P.ctx_word[band], P.instance, k, 0u);
-            const float qk = fminf(1.0f, (float)(F * (double)kScoreRate));
-            if (rs.next() < qk) {
-                vb = score_rim_dir(rs, nrm, rdir, spec);
-                const double wgt = F / (double)qk;
-                coef += wgt;
-                wcont = (float)(-wgt);
-                sdraw = rs.draw;
-                spawn = true;
-            }
-#pragma unroll
-            for (int q = 0; q < kAdMaxMat; ++q)
-                if ((uint32_t)q == mat) sacc[q] += (float)coef;
-        }
-        const uint32_t slot = block_append<kBlock>(n_out, cont, sc[2 + parity]);
+        const V3 hv = sample_hemi_wave(cont, true, rng, nrm, hl[threadIdx.x >> 6]);
         if (cont) {
-            qout.o[slot] = no;
-            qout.d[slot] = nd;
-            qout.m[slot] = nmeta;
-#pragma unroll
-            for (int q = 0; q < kAdMaxMat; ++q) {
-                if ((uint32_t)q < nm) {
-                    tout.refl(q, slot) = drefl[q];
-                    if (SCORE) tout.row(q, slot) = sacc[q];
+            const V3 d{rd.x, rd.y, rd.z};
+            const V3 rdir = bt == kRefract ? d : reflect(d, nrm);
+            const V3 vdir = blend_spec(hv, rdir, spec);
+            const uint4 next = make_uint4(rm.x, rng.draw, (uint32_t)band | (k << 8), id);
+            ro = make_float4(p.x, p.y, p.z, I);
+            rd = make_float4(vdir.x, vdir.y, vdir.z, L);
+            if (SCORE && !contn) {
+                // the direction just drawn leaves this vertex: its score, the
+                // rim flux and perhaps a continuation (after this vertex's
+                // connections, which that direction does not reach)
+                const double cdir = (double)vdir.x * (double)rdir.x + (double)vdir.y * (double)rdir.y +
+                                    (double)vdir.z * (double)rdir.z;
+                const double cr = (double)rdir.x * (double)nrm.x + (double)rdir.y * (double)nrm.y +
+                                  (double)rdir.z * (double)nrm.z;
+                const double F = score_flux(cr, (double)spec);
+                double coef = score_dlogp(cdir, (double)spec) - F;
+                Rng rs;
+                score_rng_init(rs, P.seed, rm.x, P.ctx_word[band], P.instance, k, 0u);
+                const float qk = fminf(1.0f, (float)(F * (double)kScoreRate));
+                rm = next;
+                if (rs.next() < qk) {
+                    const V3 vb = score_rim_dir(rs, nrm, rdir, spec);
+                    const double wgt = F / (double)qk;
+                    coef += wgt;
+                    wcont = (float)(-wgt);
+                    cmat = mat;
+                    kspawn = k;
+                    contn = true;
+                    mo[threadIdx.x] = ro;  // the main path waits
+                    md[threadIdx.x] = rd;
+                    mm[threadIdx.x] = rm;
+                    rd = make_float4(vb.x, vb.y, vb.z, L);
+                    rm.y = rs.draw;
                 }
+                sacc[mat * kBlock] += (float)coef;
+            } else {
+                rm = next;
             }
-            if (SCORE && contn) tout.row(nm, slot) = __uint_as_float(kspawn);
+        } else if (SCORE && contn) {
+            ro = mo[threadIdx.x];
+            rd = md[threadIdx.x];
+            rm = mm[threadIdx.x];
+            contn = false;
+        } else {
+            live = false;
         }
-        if (SCORE && !CONT) {
-            const uint32_t cs = block_append<kBlock>(co.n, spawn, sc[4 + parity]);
-            if (spawn) {
-                co.q.o[cs] = no;
-                co.q.d[cs] = make_float4(vb.x, vb.y, vb.z, L);
-                co.q.m[cs] = make_uint4(ray, sdraw, (uint32_t)band | (k << 8) | kContFlag, id);
-#pragma unroll
-                for (int q = 0; q < kAdMaxMat; ++q) {
-                    if ((uint32_t)q < nm) {
-                        co.t.refl(q, cs) = 0.0f;
-                        co.t.row(q, cs) = (uint32_t)q == mat ? wcont : 0.0f;
-                    }
-                }
-                co.t.row(nm, cs) = __uint_as_float(k);
-            }
-        }
-        n_done += i < n ? 1u : 0u;
     }
-    stat_add(stats, ST_SEGMENTS, n_done);
-}
-
-// Visibility of the local adjoint's connection requests (Scene::Connect,
-// src/Scene.cpp:84-96): the lane-refilling any-hit walk of k_shadow_f; a
-// visible request adds its weights to the gradient of its instance and band.
-template <int WIDTH, bool BATCH>
-__global__ void __launch_bounds__(kBlock) k_adj_vis(const InstDev* __restrict__ inst, int* gstack, uint32_t gthreads,
-                                                     AdjShadowQ aq, const uint32_t* __restrict__ n_aq, AdjArgs A0,
-                                                     const AdjArgs* __restrict__ adj,
-                                                     unsigned long long* __restrict__ stats, Fetch fetch) {
-    constexpr int LDS = 16;
-    __shared__ int lds[LDS * kBlock];
-    const uint32_t n = *n_aq;
-    const uint32_t gtid = blockIdx.x * kBlock + threadIdx.x;
-    const uint32_t lane = lane_id();
-    uint32_t nvis = 0, ntri = 0, nsh = 0;
-    Walker<LDS, kBlock, WIDTH, true, false> w(lds + threadIdx.x, gstack, gtid, gthreads);
-    Traversal T = make_trav(inst[0], gstack, gthreads);
-    double g_refl[kAdMaxMat], g_spec[kAdMaxMat];
-#pragma unroll
-    for (int q = 0; q < kAdMaxMat; ++q) g_refl[q] = g_spec[q] = 0.0;
-    uint32_t key = 0xFFFFFFFFu;  // instance of the accumulated partials
-    int kband = -1;
-    Claim claim(n, gtid, gridDim.x * blockDim.x, fetch);
-    uint32_t refill = fetch.refill;
-    bool pending = false;  // a visible request not yet added
-    uint32_t slot = 0;
-    for (;;) {
-        const uint64_t idle = __ballot(w.idle());
-        if ((uint32_t)__popcll(idle) >= refill) {
-            if (pending) {
-                const uint4 m = aq.m[slot];
-                const uint32_t id = BATCH ? m.y : 0u;
-                const int band = (int)((m.x >> 8) & 0xFFu);
-                if (BATCH && key != 0xFFFFFFFFu && (id != key || band != kband)) {
-                    // a batch lane moving to another instance or band hands its partials on
-                    const AdjArgs& A = adj[key];
-                    double* gk = A.grad_copy();
-#pragma unroll
-                    for (int q = 0; q < kAdMaxMat; ++q) {
-                        if ((uint32_t)q < A.n_mat) {
-                            if (g_refl[q] != 0.0) atomicAdd(gk + ((size_t)kband * 2 + 0) * A.n_mat + q, g_refl[q]);
-                            if (g_spec[q] != 0.0) atomicAdd(gk + ((size_t)kband * 2 + 1) * A.n_mat + q, g_spec[q]);
-                        }
-                        g_refl[q] = g_spec[q] = 0.0;
-                    }
-                }
-                key = id;
-                kband = band;
-                const float4 w0 = aq.w[4 * (size_t)slot], w1 = aq.w[4 * (size_t)slot + 1];
-                const float4 w2 = aq.w[4 * (size_t)slot + 2], w3 = aq.w[4 * (size_t)slot + 3];
-                const float wq[8] = {w0.x, w0.y, w0.z, w0.w, w1.x, w1.y, w1.z, w1.w};
-                const float wsq[8] = {w2.x, w2.y, w2.z, w2.w, w3.x, w3.y, w3.z, w3.w};
-#pragma unroll
-                for (int q = 0; q < kAdMaxMat; ++q) {
-                    g_refl[q] += (double)wq[q];
-                    g_spec[q] += (double)wsq[q];
-                }
-                pending = false;
-            }
-            const uint32_t mine = claim.take(fetch, idle, lane);
-            if (mine != 0xFFFFFFFFu) {
-                slot = mine;
-                ++nsh;
-                const float4 pw = aq.p[mine];
-                const uint4 m = aq.m[mine];
-                const uint32_t id = BATCH ? m.y : 0u;
-                if (BATCH) T = make_trav(inst[id], gstack, gthreads);
-                const RecParams& R = inst[id].P.rec[m.x & 0xFFu];
-                const V3 p{pw.x, pw.y, pw.z};
-                w.start(T, p, sub(V3{R.px, R.py, R.pz}, p), 0.0f);
-                pending = w.idle();  // empty scene: visible
-            }
-            // the loop is left by the whole wave at once
-            if (idle == ~0ull && __ballot(mine != 0xFFFFFFFFu) == 0) break;
-            if (claim.exhausted()) refill = 64u;
-        }
-        if (w.step(T, nvis, ntri)) pending = !w.found();
-    }
-    stat_add(stats, ST_SHADOW, nsh);
-    if (!BATCH) {
-        __shared__ double red[kBlock / 64][2 * kAdMaxMat];
-        block_grad_flush(A0, kband, g_refl, g_spec, &red[0][0]);
-        return;
-    }
-    // what is left, reduced per instance and band present in the wave
+    // what is left, summed over the lanes of the wave that hold the same
+    // instance and band
     uint64_t todo = __ballot(key != 0xFFFFFFFFu);
     while (todo) {
         const int leader = __ffsll((unsigned long long)todo) - 1;
         const uint32_t lk = __shfl(key, leader);
         const int lb = __shfl(kband, leader);
         const bool mine = key == lk && kband == lb;
-        const uint32_t nmk = adj[lk].n_mat;
-        double* gk = adj[lk].grad_copy();
+        const AdjArgs& A = BATCH ? adj[lk] : A0;
+        double* gk = A.grad_copy() + (size_t)lb * 2 * A.n_mat;
 #pragma unroll
-        for (int q = 0; q < kAdMaxMat; ++q) {
-            if ((uint32_t)q >= nmk) break;
-            const double sr = wave_sum_d(mine ? g_refl[q] : 0.0);
-            const double ss = wave_sum_d(mine ? g_spec[q] : 0.0);
+        for (int m = 0; m < kAdMaxMat; ++m) {
+            if ((uint32_t)m >= A.n_mat) break;
+            const double sr = wave_sum_d(mine ? g_refl[m] : 0.0);
+            const double ss = wave_sum_d(mine ? g_spec[m] : 0.0);
             if (lane == 0) {
-                if (sr != 0.0) atomicAdd(gk + ((size_t)lb * 2 + 0) * nmk + q, sr);
-                if (ss != 0.0) atomicAdd(gk + ((size_t)lb * 2 + 1) * nmk + q, ss);
+                add_grad(gk + m, sr);
+                add_grad(gk + A.n_mat + m, ss);
             }
         }
         todo &= ~__ballot(mine);
@@ -4102,33 +4001,6 @@ ear_status run_backward_batch(Ctx* c, uint32_t n_items, DeviceScene* const* scen
     }
     const ear_tuning& tu = c->tuning;
     const uint32_t chunk = tu.ray_chunk ? tu.ray_chunk : (1u << 23);
-    uint64_t rays_any = 0;
-    for (uint32_t i = 0; i < n_items; ++i) rays_any = std::max<uint64_t>(rays_any, descs[i]->n_rays);
-    uint64_t rays_band_max = 0;
-    for (int b = 0; b < 3; ++b) {
-        uint64_t t = 0;
-        for (uint32_t i = 0; i < n_items; ++i)
-            if ((inst[i].P.band_mask >> b) & 1u) t += descs[i]->n_rays;
-        rays_band_max = std::max(rays_band_max, t);
-    }
-    const uint32_t cap = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(chunk, rays_band_max));
-    hipStream_t st = c->stream;
-    DevBuf qo[2] = {DevBuf(c), DevBuf(c)}, qd[2] = {DevBuf(c), DevBuf(c)}, qm[2] = {DevBuf(c), DevBuf(c)};
-    DevBuf tt[2] = {DevBuf(c), DevBuf(c)}, tr[2] = {DevBuf(c), DevBuf(c)};
-    DevBuf hits(c), counters(c), stats(c), gs(c), dinst(c), dsegs(c), dsegoff(c), dplan(c), dadj_s(c), dadj_a(c),
-        dgrad(c), dargs(c), sqp(c), sqm(c);
-    for (int k = 0; k < 2; ++k) {
-        TRY(qo[k].alloc((size_t)cap * 16));
-        TRY(qd[k].alloc((size_t)cap * 16));
-        TRY(qm[k].alloc((size_t)cap * 16));
-        TRY(tt[k].alloc((size_t)cap * nm_max * 8 * 4));
-        TRY(tr[k].alloc((size_t)cap * nm_max * 4));
-    }
-    TRY(counters.alloc(32));
-    TRY(stats.alloc(ST_N * 8 * kStatCopies));
-    TRY(sqp.alloc(16));
-    TRY(sqm.alloc(16));
-    // connection requests of the local adjoint (one per ray and recorder)
     uint32_t n_local = 0, n_score = 0;
     for (uint32_t i = 0; i < n_items; ++i) {
         n_local += (inst[i].P.flags & EAR_FLAG_ADJ_LOCAL) ? 1u : 0u;
@@ -4139,33 +4011,36 @@ ear_status run_backward_batch(Ctx* c, uint32_t n_items, DeviceScene* const* scen
         return EAR_ERR_INVALID_ARGUMENT;
     }
     const bool all_score = n_score == n_items;
-    const bool all_local = all_score || n_local == n_items;  // the per-vertex kernels
-    DevBuf aqp(c), aqm(c), aqw(c), segv(c);
-    // the score form's continuations: traced one bounce per main bounce in
-    // their own queues (qc), then to their ends after the chunk's main rays;
-    // room for four chunks (about the most that are alive at once: spawns
-    // build up as ~0.05 F per live ray and bounce), a drain when full
-    const uint32_t cap_c = all_score ? (uint32_t)std::min<uint64_t>(4ull * cap, 1ull << 25) : 1u;
-    const uint32_t cap_q = std::max(cap, cap_c);  // rays of one bounce: the chunk or a drain
-    TRY(hits.alloc((size_t)cap_q * 8));
-    const size_t cap_aq = all_local ? (size_t)cap_q * std::max<uint32_t>(1, max_rec) : 1;
-    TRY(aqp.alloc(cap_aq * 16));
-    TRY(aqm.alloc(cap_aq * 16));
-    TRY(aqw.alloc(cap_aq * 64));
-    DevBuf qco[2] = {DevBuf(c), DevBuf(c)}, qcd[2] = {DevBuf(c), DevBuf(c)}, qcm[2] = {DevBuf(c), DevBuf(c)};
-    DevBuf tct[2] = {DevBuf(c), DevBuf(c)}, tcr[2] = {DevBuf(c), DevBuf(c)}, cntc(c);
-    for (int k = 0; k < 2; ++k) {
-        TRY(qco[k].alloc((size_t)cap_c * 16));
-        TRY(qcd[k].alloc((size_t)cap_c * 16));
-        TRY(qcm[k].alloc((size_t)cap_c * 16));
-        TRY(tct[k].alloc((size_t)cap_c * (nm_max + 1) * 4));
-        TRY(tcr[k].alloc((size_t)cap_c * nm_max * 4));
+    const bool all_local = all_score || n_local == n_items;  // one launch per chunk of rays (k_adj_paths)
+    // the queue holds a chunk of the rays of one band, or of all of them
+    uint64_t rays_band_max = 0, rays_all = 0;
+    for (int b = 0; b < 3; ++b) {
+        uint64_t t = 0;
+        for (uint32_t i = 0; i < n_items; ++i)
+            if ((inst[i].P.band_mask >> b) & 1u) t += descs[i]->n_rays;
+        rays_band_max = std::max(rays_band_max, t);
+        rays_all += t;
     }
-    TRY(cntc.alloc(8));
-    EAR_HIP_TRY(c, hipMemsetAsync(cntc.p, 0, cntc.n, st));
-    TRY(segv.alloc(kMaxSeg * kSegStride * 4));
-    EAR_HIP_TRY(c, hipMemsetAsync(segv.p, 0, segv.n, st));
-    const AdjShadowQ AQ{aqp.as<float4>(), aqm.as<uint4>(), aqw.as<float4>()};
+    const uint32_t cap =
+        (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(chunk, all_local ? rays_all : rays_band_max));
+    hipStream_t st = c->stream;
+    DevBuf qo[2] = {DevBuf(c), DevBuf(c)}, qd[2] = {DevBuf(c), DevBuf(c)}, qm[2] = {DevBuf(c), DevBuf(c)};
+    DevBuf tt[2] = {DevBuf(c), DevBuf(c)}, tr[2] = {DevBuf(c), DevBuf(c)};
+    DevBuf hits(c), counters(c), stats(c), gs(c), dinst(c), dsegs(c), dsegoff(c), dplan(c), dadj_s(c), dadj_a(c),
+        dgrad(c), dargs(c), sqp(c), sqm(c);
+    for (int k = 0; k < (all_local ? 1 : 2); ++k) {
+        TRY(qo[k].alloc((size_t)cap * 16));
+        TRY(qd[k].alloc((size_t)cap * 16));
+        TRY(qm[k].alloc((size_t)cap * 16));
+        if (all_local) continue;
+        TRY(tt[k].alloc((size_t)cap * nm_max * 8 * 4));
+        TRY(tr[k].alloc((size_t)cap * nm_max * 4));
+    }
+    TRY(counters.alloc(32));
+    TRY(stats.alloc(ST_N * 8 * kStatCopies));
+    TRY(sqp.alloc(16));
+    TRY(sqm.alloc(16));
+    if (!all_local) TRY(hits.alloc((size_t)cap * 8));
     // static closest-hit traversal by default (the replayed bands run one
     // at a time, with fewer rays in flight than the forward's, where the
     // refill bookkeeping does not pay); the refilling one on request
@@ -4183,12 +4058,18 @@ ear_status run_backward_batch(Ctx* c, uint32_t n_items, DeviceScene* const* scen
     const uint32_t cap_e = (uint32_t)c->num_cus * (uint32_t)std::max(1, resident_blocks((const void*)fe, 256));
     const uint32_t gmax = persistent_grid(c, 0xFFFFFFFFu, waves);
     // every thread of either traversal launch owns one overflow stack
-    const uint32_t gthreads = std::max(cap_e * 256u, gmax * (uint32_t)kBlock);
-    TRY(gs.alloc((size_t)(kStackDepth - kLdsMin) * gthreads * 4));
+    using PathsFn = void (*)(const InstDev*, int*, uint32_t, Queue, const uint32_t*, uint32_t, AdjArgs, const AdjArgs*, Fetch);
+    const PathsFn paths = width == 4 ? (batch ? (all_score ? (PathsFn)k_adj_paths<4, true, true> : (PathsFn)k_adj_paths<4, true, false>)
+                                              : (all_score ? (PathsFn)k_adj_paths<4, false, true> : (PathsFn)k_adj_paths<4, false, false>))
+                                     : (batch ? (all_score ? (PathsFn)k_adj_paths<2, true, true> : (PathsFn)k_adj_paths<2, true, false>)
+                                              : (all_score ? (PathsFn)k_adj_paths<2, false, true> : (PathsFn)k_adj_paths<2, false, false>));
+    const uint32_t g_paths = (uint32_t)c->num_cus * (uint32_t)std::max(1, resident_blocks((const void*)paths, kBlock));
+    const uint32_t gthreads = all_local ? g_paths * (uint32_t)kBlock : std::max(cap_e * 256u, gmax * (uint32_t)kBlock);
+    TRY(gs.alloc((size_t)(kStackDepth - (all_local ? kAdjLds : kLdsMin)) * gthreads * 4));
     TRY(dinst.alloc(sizeof(InstDev) * n_items));
-    TRY(dsegs.alloc(sizeof(GenSeg) * n_items));
-    TRY(dsegoff.alloc(4 * (size_t)n_items));
-    TRY(dplan.alloc(8));
+    TRY(dsegs.alloc(sizeof(GenSeg) * 3 * (size_t)n_items));
+    TRY(dsegoff.alloc(4 * 3 * (size_t)n_items));
+    TRY(dplan.alloc(12));
     const uint32_t grad_n = 3 * 2 * nm_max * n_items;  // one copy
     TRY(dgrad.alloc(sizeof(double) * (size_t)grad_n * kGradCopies));
     TRY(dargs.alloc(sizeof(AdjArgs) * n_items));
@@ -4249,91 +4130,55 @@ ear_status run_backward_batch(Ctx* c, uint32_t n_items, DeviceScene* const* scen
                   Queue{qo[1].as<float4>(), qd[1].as<float4>(), qm[1].as<uint4>()}};
     Tangents T[2] = {Tangents{tt[0].as<float>(), tr[0].as<float>(), cap},
                      Tangents{tt[1].as<float>(), tr[1].as<float>(), cap}};
-    Queue qc[2] = {Queue{qco[0].as<float4>(), qcd[0].as<float4>(), qcm[0].as<uint4>()},
-                   Queue{qco[1].as<float4>(), qcd[1].as<float4>(), qcm[1].as<uint4>()}};
-    Tangents Tc[2] = {Tangents{tct[0].as<float>(), tcr[0].as<float>(), cap_c},
-                      Tangents{tct[1].as<float>(), tcr[1].as<float>(), cap_c}};
-    uint32_t* ncc = cntc.as<uint32_t>();
-    int ci = 0;              // the continuations' input buffer
-    uint32_t n_cont = 0;     // continuations waiting there
-    bool cont_live = false;  // any may be waiting (a main bounce has run since the last drain)
-    uint32_t pinned_c[2];
     const ShadowQ SQ{sqp.as<float4>(), sqm.as<float4>()};
     const AdjArgs A0 = args[0];
     const AdjArgs* dA = dargs.as<AdjArgs>();
-    // the visibility kernel: lane refilling over the request queue
-    using VisFn = void (*)(const InstDev*, int*, uint32_t, AdjShadowQ, const uint32_t*, AdjArgs, const AdjArgs*,
-                           unsigned long long*, Fetch);
-    const VisFn fv = width == 4 ? (batch ? k_adj_vis<4, true> : k_adj_vis<4, false>)
-                                : (batch ? k_adj_vis<2, true> : k_adj_vis<2, false>);
-    const uint32_t cap_v = (uint32_t)c->num_cus * (uint32_t)std::max(1, resident_blocks((const void*)fv, kBlock));
-    // grids of the per-vertex shading kernels (no walk inside them, so no
-    // overflow stacks to cover) and of the continuations' shading
-    const uint32_t cap_sl =
-        rounds_cap(c,
-                   batch ? (all_score ? (const void*)k_shade_adl<true, true> : (const void*)k_shade_adl<true, false>)
-                         : (all_score ? (const void*)k_shade_adl<false, true> : (const void*)k_shade_adl<false, false>),
-                   tu.waves_per_cu, kBlock);
-    const uint32_t cap_sc = rounds_cap(
-        c, batch ? (const void*)k_shade_adl<true, true, true> : (const void*)k_shade_adl<false, true, true>,
-        tu.waves_per_cu, kBlock);
-    const Fetch fq_v{segv.as<uint32_t>(), tu.refill ? tu.refill : 24u, tu.fetch_chunk, nseg};
-    // one bounce of the per-vertex adjoint (local or score form): closest
-    // hits of queue qi, the shade (continuing rays into qo, continuations
-    // into co), the visibility of the connection requests
-    auto adl_bounce = [&](const Queue& qi, uint32_t* ni, const Tangents& ti, const Queue& qo, uint32_t* no,
-                          const Tangents& to, const ContOut& co, uint32_t n_now, uint32_t gsd, uint32_t ge,
-                          bool conts) {
-        hipLaunchKernelGGL(fe, dim3(ge), dim3(256), 0, st, di, gs.as<int>(), gthreads, qi, (const uint32_t*)ni,
-                           hits.as<int2>(), stp, fq_e);
-        if (fetch_e) k_reset_iter<<<1, 64, 0, st>>>(cnt, 0u, segc.as<uint32_t>(), nseg);
-        if (conts) {
-            if (batch)
-                k_shade_adl<true, true, true><<<gsd, kBlock, 0, st>>>(di, qi, ni, hits.as<int2>(), ti, qo, no, to,
-                                                                      AQ, cnt + 2, max_rec, A0, dA, co, stp);
-            else
-                k_shade_adl<false, true, true><<<gsd, kBlock, 0, st>>>(di, qi, ni, hits.as<int2>(), ti, qo, no, to,
-                                                                       AQ, cnt + 2, max_rec, A0, dA, co, stp);
-        } else if (batch) {
-            if (all_score)
-                k_shade_adl<true, true><<<gsd, kBlock, 0, st>>>(di, qi, ni, hits.as<int2>(), ti, qo, no, to, AQ,
-                                                                cnt + 2, max_rec, A0, dA, co, stp);
-            else
-                k_shade_adl<true, false><<<gsd, kBlock, 0, st>>>(di, qi, ni, hits.as<int2>(), ti, qo, no, to, AQ,
-                                                                 cnt + 2, max_rec, A0, dA, co, stp);
-        } else {
-            if (all_score)
-                k_shade_adl<false, true><<<gsd, kBlock, 0, st>>>(di, qi, ni, hits.as<int2>(), ti, qo, no, to, AQ,
-                                                                 cnt + 2, max_rec, A0, dA, co, stp);
-            else
-                k_shade_adl<false, false><<<gsd, kBlock, 0, st>>>(di, qi, ni, hits.as<int2>(), ti, qo, no, to, AQ,
-                                                                  cnt + 2, max_rec, A0, dA, co, stp);
+    if (all_local) {
+        // every (instance, band) context is a run of rays (as many runs at a
+        // time as 32-bit ray numbers reach over); a chunk of rays is emitted
+        // and carried to its paths' ends at a time
+        uint32_t dense = 1;
+        std::vector<GenSeg> todo;
+        for (uint32_t i = 0; i < n_items; ++i) {
+            if (1.0 < inst[i].P.cutoff || inst[i].P.max_bounces == 0) dense = 0;
+            for (uint32_t b = 0; b < 3; ++b)
+                if (((inst[i].P.band_mask >> b) & 1u) && descs[i]->n_rays != 0)
+                    todo.push_back(GenSeg{i, b, 0, descs[i]->n_rays});
         }
-        const uint32_t n_req = (uint32_t)std::min<size_t>(cap_aq, (size_t)n_now * max_rec);
-        hipLaunchKernelGGL(fv, dim3(grid_for(n_req, cap_v, kBlock)), dim3(kBlock), 0, st, di, gs.as<int>(), gthreads,
-                           AQ, (const uint32_t*)(cnt + 2), A0, dA, stp, fq_v);
-        k_reset_iter<<<1, 64, 0, st>>>(cnt, 0u, segv.as<uint32_t>(), nseg);
-        k_reset2<<<1, 64, 0, st>>>(ni, cnt + 2);
-    };
-    // the waiting continuations traced to their ends (they spawn nothing,
-    // so a queue never grows within a drain)
-    auto drain = [&]() -> ear_status {
-        cont_live = false;
-        while (n_cont > 0) {
-            const uint32_t gsd = grid_for(n_cont, cap_sc, kBlock);
-            const uint32_t ge = grid_for(n_cont, cap_e, 256);
-            for (int gi = 0; gi < 4; ++gi) {
-                adl_bounce(qc[ci], ncc + ci, Tc[ci], qc[1 - ci], ncc + (1 - ci), Tc[1 - ci],
-                           ContOut{qc[ci], ncc + ci, Tc[ci]}, n_cont, gsd, ge, true);
-                ci = 1 - ci;
+        for (size_t s0 = 0; s0 < todo.size();) {
+            std::vector<uint32_t> off;
+            uint64_t total = 0;
+            size_t s1 = s0;
+            for (; s1 < todo.size() && (s1 == s0 || total + todo[s1].count <= 0xFFFFFFFFull); ++s1) {
+                off.push_back((uint32_t)total);
+                total += todo[s1].count;
             }
-            EAR_HIP_TRY(c, hipMemcpyAsync(pinned_c, ncc, 8, hipMemcpyDeviceToHost, st));
-            EAR_HIP_TRY(c, hipStreamSynchronize(st));
-            n_cont = pinned_c[ci];
+            EAR_HIP_TRY(c, hipMemcpyAsync(dsegs.p, todo.data() + s0, sizeof(GenSeg) * (s1 - s0), hipMemcpyHostToDevice, st));
+            EAR_HIP_TRY(c, hipMemcpyAsync(dsegoff.p, off.data(), 4 * off.size(), hipMemcpyHostToDevice, st));
+            for (uint64_t r0 = 0; r0 < total; r0 += cap) {
+                const uint32_t n_chunk = (uint32_t)std::min<uint64_t>(cap, total - r0);
+                const uint32_t plan[3] = {(uint32_t)r0, n_chunk, 0u}, n_live = dense ? n_chunk : 0u;
+                EAR_HIP_TRY(c, hipMemcpyAsync(dplan.p, plan, 12, hipMemcpyHostToDevice, st));
+                EAR_HIP_TRY(c, hipMemcpyAsync(cnt, &n_live, 4, hipMemcpyHostToDevice, st));
+                const uint32_t g = persistent_grid(c, n_chunk, waves);
+                if (batch)
+                    k_generate<true><<<g, kBlock, 0, st>>>(di, dsegs.as<GenSeg>(), dsegoff.as<uint32_t>(),
+                                                           (uint32_t)off.size(), n_chunk, dplan.as<uint32_t>(), max_rec,
+                                                           0u, dense, q[0], cnt, SQ, cnt + 2, stp);
+                else
+                    k_generate<false><<<g, kBlock, 0, st>>>(di, dsegs.as<GenSeg>(), dsegoff.as<uint32_t>(),
+                                                            (uint32_t)off.size(), n_chunk, dplan.as<uint32_t>(), max_rec,
+                                                            0u, dense, q[0], cnt, SQ, cnt + 2, stp);
+                hipLaunchKernelGGL(paths, dim3(g_paths), dim3(kBlock), 0, st, di, gs.as<int>(), gthreads, q[0],
+                                   (const uint32_t*)cnt, max_rec, A0, dA, fq_e);
+                k_reset_iter<<<1, 64, 0, st>>>(cnt, 0u, segc.as<uint32_t>(), nseg);
+                EAR_HIP_TRY(c, hipGetLastError());
+                EAR_HIP_TRY(c, hipStreamSynchronize(st));  // plan, n_live and off leave scope
+            }
+            s0 = s1;
         }
-        return EAR_OK;
-    };
-    for (uint32_t band = 0; band < 3; ++band) {
+    }
+    for (uint32_t band = 0; !all_local && band < 3; ++band) {
         // this band's contexts as runs of rays
         std::vector<GenSeg> segs;
         std::vector<uint32_t> off;
@@ -4359,7 +4204,7 @@ ear_status run_backward_batch(Ctx* c, uint32_t n_items, DeviceScene* const* scen
                 k_generate<false><<<persistent_grid(c, n_chunk, waves), kBlock, 0, st>>>(
                     di, dsegs.as<GenSeg>(), dsegoff.as<uint32_t>(), (uint32_t)segs.size(), n_chunk,
                     dplan.as<uint32_t>(), max_rec, 0u, 0u, q[0], cnt + 0, SQ, cnt + 2, stp);
-            if (!all_local || all_score) k_zero_f32<<<1024, 256, 0, st>>>(T[0].t, (size_t)cap * nm_max * 8);
+            k_zero_f32<<<1024, 256, 0, st>>>(T[0].t, (size_t)cap * nm_max * 8);
             k_zero_f32<<<1024, 256, 0, st>>>(T[0].r, (size_t)cap * nm_max);
             EAR_HIP_TRY(c, hipMemcpyAsync(pinned, cnt, 12, hipMemcpyDeviceToHost, st));
             EAR_HIP_TRY(c, hipStreamSynchronize(st));
@@ -4370,33 +4215,12 @@ ear_status run_backward_batch(Ctx* c, uint32_t n_items, DeviceScene* const* scen
             // within a chunk, so grids sized at a group's start cover it
             uint32_t k = 1;
             while (k <= max_bounces && n_live > 0) {
-              uint32_t group = std::min<uint32_t>(4u, max_bounces - k + 1);
-              if (all_score) {
-                  // every bounce may append one continuation per live ray, and
-                  // the continuations' own bounce never adds any
-                  if (cap_c - n_cont < n_live) TRY(drain());
-                  group = std::min<uint32_t>(group, (cap_c - n_cont) / n_live);
-              }
+              const uint32_t group = std::min<uint32_t>(4u, max_bounces - k + 1);
               // k_shade_ad walks inside: its grid stays within the overflow stacks' gmax
-              const uint32_t gsd = all_local ? grid_for(n_live, cap_sl, kBlock) : persistent_grid(c, n_live, waves);
+              const uint32_t gsd = persistent_grid(c, n_live, waves);
               const uint32_t ge = grid_for(n_live, cap_e, 256);
-              const uint32_t n_cmax = all_score ? n_cont + group * n_live : 0u;
-              const uint32_t gsd_c = grid_for(std::max(1u, n_cmax), cap_sc, kBlock);
-              const uint32_t ge_c = grid_for(std::max(1u, n_cmax), cap_e, 256);
               for (uint32_t gi = 0; gi < group; ++gi, ++k) {
-                if (all_local) {
-                    // the main bounce: its spawns join the continuations' next input
-                    adl_bounce(q[cur], cnt + cur, T[cur], q[1 - cur], cnt + (1 - cur), T[1 - cur],
-                               ContOut{qc[1 - ci], ncc + (1 - ci), Tc[1 - ci]}, n_live, gsd, ge, false);
-                    if (all_score) {
-                        // one bounce of the waiting continuations, beside the main rays
-                        if (cont_live)
-                            adl_bounce(qc[ci], ncc + ci, Tc[ci], qc[1 - ci], ncc + (1 - ci), Tc[1 - ci],
-                                       ContOut{qc[ci], ncc + ci, Tc[ci]}, n_cmax, gsd_c, ge_c, true);
-                        cont_live = true;
-                        ci = 1 - ci;
-                    }
-                } else {
+                {
                     hipLaunchKernelGGL(fe, dim3(ge), dim3(256), 0, st, di, gs.as<int>(), gthreads, q[cur],
                                        (const uint32_t*)(cnt + cur), hits.as<int2>(), stp, fq_e);
                     if (fetch_e) k_reset_iter<<<1, 64, 0, st>>>(cnt, 0u, segc.as<uint32_t>(), nseg);
@@ -4420,12 +4244,9 @@ ear_status run_backward_batch(Ctx* c, uint32_t n_items, DeviceScene* const* scen
                 cur = 1 - cur;
               }
               EAR_HIP_TRY(c, hipMemcpyAsync(pinned, cnt, 12, hipMemcpyDeviceToHost, st));
-              if (all_score) EAR_HIP_TRY(c, hipMemcpyAsync(pinned_c, ncc, 8, hipMemcpyDeviceToHost, st));
               EAR_HIP_TRY(c, hipStreamSynchronize(st));
               n_live = pinned[cur];
-              if (all_score) n_cont = pinned_c[ci];
             }
-            if (all_score) TRY(drain());
             k_reset2<<<1, 64, 0, st>>>(cnt + 0, cnt + 1);
             EAR_HIP_TRY(c, hipGetLastError());
         }
