@@ -259,7 +259,7 @@ def kernel_rooflines(acc, ist, info, traffic_dir, steps):
         material) + 16 (material row) + 48 x (segments that continue) + 32 x
         (shadow requests written)
       k_shadow_f per shadow query: 32 (request) + B V_sh + 36 T_sh, plus per
-        ramp 3 x 16 (128-bit points) with direct atomics, or with the
+        ramp 16 (its 128-bit point) with direct atomics, or with the
         time-tiled splat 4 per record slot + 8 per record
     B = 64 bytes per node visit.  `traffic` is rocprofv3's FETCH_SIZE +
     WRITE_SIZE per launch of that kernel (scaled by a plain copy), where
@@ -279,7 +279,7 @@ def kernel_rooflines(acc, ist, info, traffic_dir, steps):
         "k_extend_f": (24 + 8 + B * V + 36 * T, qe, acc["extend_ms"], acc["extend_launches"], "closest-hit query"),
         "k_shade": (48 + 8 + 16 + 16 + 48 * cont + 32 * qs / qe, qe, acc["shade_ms"], acc["extend_launches"],
                     "shaded segment"),
-        "k_shadow_f": (32 + B * Vs + 36 * Ts + (4 * stride + 8 * ramps_per_q if tiled else 48 * ramps_per_q), qs,
+        "k_shadow_f": (32 + B * Vs + 36 * Ts + (4 * stride + 8 * ramps_per_q if tiled else 16 * ramps_per_q), qs,
                        acc["shadow_ms"], acc["shadow_launches"], "shadow query"),
     }
     out = {}
@@ -306,11 +306,11 @@ def kernel_rooflines(acc, ist, info, traffic_dir, steps):
     # the whole render (all kernels, trace_ms): bytes per segment with every
     # shadow query and ramp of the render
     seg = max(1, acc["segments"])
-    b_seg = (96 + 20 + B * (V + Vs * qs / seg) + 36 * (T + Ts * qs / seg) + 48 * acc["shadow_ramps"] / seg)
+    b_seg = (96 + 20 + B * (V + Vs * qs / seg) + 36 * (T + Ts * qs / seg) + 16 * acc["shadow_ramps"] / seg)
     ach = b_seg * seg / max(1e-9, acc["trace_ms"] * 1e-3) / 1e9
     render_roof = {"bytes_per_segment": round(b_seg, 1), "achieved": round(ach, 1), "peak": HBM_PEAK_GBS,
                    "unit": "GB/s", "frac": round(ach / HBM_PEAK_GBS, 4),
-                   "note": "96 ray state + 20 material + 64 (V + V_sh) + 36 (T + T_sh) + 48 per ramp, per segment"}
+                   "note": "96 ray state + 20 material + 64 (V + V_sh) + 36 (T + T_sh) + 16 per ramp, per segment"}
     return out, render_roof
 
 
