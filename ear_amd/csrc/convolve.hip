@@ -10,7 +10,7 @@
 // convolution unchanged), and both products are summed in the frequency
 // domain, so one inverse transform serves both terms.
 //
-// Up to 2^22 samples (95 s) the transforms are the three kernels below, in
+// Up to 2^22 samples (95 s) the transforms are the kernels below, in
 // binary64; longer ones are batched hipFFT real transforms.  What bounded a
 // call was the library's plan, made and dropped with its code objects on every
 // call: 24 of 26 ms for 3 s of response and 10 s of faded sound, whose kernels
@@ -43,8 +43,9 @@ __global__ void k_spectra_mul(const float2* __restrict__ X, uint32_t nc, uint32_
 }
 
 // ---------------------------------------------------------------------------
-// The convolution in three kernels.  A track and its signal are the real and
+// The convolution.  A track and its signal are the real and
 // imaginary parts of one sequence z of L = N1 N2 values.  Index n = n1 N2 + n2:
+//   k_conv_peaks    the operands' largest samples (see Level)
 //   k_conv_columns  the N1-point transforms down the columns n2, times
 //                   e^(-2 pi i k1 n2 / L); reads the real inputs, writes z
 //   k_conv_rows     the N2-point transforms along the rows k1 (frequency
@@ -64,9 +65,61 @@ constexpr int kConvThreads = 256;
 constexpr int kConvValues = 4096;
 constexpr int kConvMinLog = 12, kConvMaxLog = 22;  // N1 and N2 are 2^6 .. 2^11
 
+struct ConvTerm {
+    const float* track;
+    const float* signal;
+    uint32_t n_track, n_signal;
+};
+
 __device__ __forceinline__ double2 cmul(double2 a, double2 b) {
     return make_double2(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x);
 }
+// The rounding of a transform is relative to the largest of what it holds, so a
+// track and its signal go into one sequence each divided by the power of two
+// 2^e that brings its largest sample into [1/2, 1) (exact); the product is
+// scaled back before the terms are summed.  Without it a response 1e-12 of its
+// sound kept 3 digits.  A term with nothing in its track or signal adds nothing.
+struct Level {
+    uint32_t bits;  // of the largest |sample|; above infinity's: a NaN
+    __device__ __forceinline__ bool silent() const { return bits == 0; }
+    __device__ __forceinline__ bool finite() const { return bits < 0x7F800000u; }
+    __device__ __forceinline__ int exponent() const {
+        if (silent() || !finite()) return 0;
+        return bits >> 23 ? (int)(bits >> 23) - 126 : (32 - __clz((int)bits)) - 149;
+    }
+};
+constexpr int kPeakBlocks = 64;  // partial maxima of an operand: one a lane
+
+// block (b, 2 term + {0 track, 1 signal}): the largest |sample| of every
+// kPeakBlocks-th run of the operand
+__global__ void __launch_bounds__(kConvThreads) k_conv_peaks(ConvTerm t0, ConvTerm t1, uint32_t* __restrict__ peaks) {
+    const ConvTerm t = blockIdx.y >> 1 ? t1 : t0;
+    const float* x = blockIdx.y & 1u ? t.signal : t.track;
+    const uint32_t n = blockIdx.y & 1u ? t.n_signal : t.n_track;
+    uint32_t m = 0;
+    for (uint32_t i = blockIdx.x * kConvThreads + threadIdx.x; i < n; i += kPeakBlocks * kConvThreads)
+        m = max(m, __float_as_uint(x[i]) & 0x7FFFFFFFu);
+    for (int o = 32; o; o >>= 1) m = max(m, (uint32_t)__shfl_xor((int)m, o));
+    __shared__ uint32_t wave[kConvThreads / 64];
+    if ((threadIdx.x & 63u) == 0) wave[threadIdx.x >> 6] = m;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int w = 1; w < kConvThreads / 64; ++w) m = max(m, wave[w]);
+        peaks[blockIdx.y * kPeakBlocks + blockIdx.x] = m;
+    }
+}
+
+// the whole wave calls it
+__device__ __forceinline__ Level level_of(const uint32_t* peaks, uint32_t operand) {
+    uint32_t m = peaks[operand * kPeakBlocks + (threadIdx.x & 63u)];
+    for (int o = 32; o; o >>= 1) m = max(m, (uint32_t)__shfl_xor((int)m, o));
+    return Level{(uint32_t)__builtin_amdgcn_readfirstlane((int)m)};
+}
+// (silence beside a NaN or an infinity is carried on: it makes NaNs)
+__device__ __forceinline__ bool nothing(Level a, Level b) {
+    return (a.silent() && b.finite()) || (b.silent() && a.finite());
+}
+
 // e^(2 pi i num / 2^lg); num / 2^lg is exact
 __device__ __forceinline__ double2 unit_root(double num, int lg) {
     double s, c;
@@ -135,25 +188,23 @@ __device__ __forceinline__ void fill_roots(double2* tw, int lg) {
     for (int j = (int)threadIdx.x; j < (1 << lg); j += kConvThreads) tw[j] = unit_root(-(double)j, lg);
 }
 
-struct ConvTerm {
-    const float* track;
-    const float* signal;
-    uint32_t n_track, n_signal;
-};
-
 // block: kConvValues >> lg1 columns of term blockIdx.y
 __global__ void __launch_bounds__(kConvThreads) k_conv_columns(ConvTerm t0, ConvTerm t1, int lg1, int lg2,
+                                                               const uint32_t* __restrict__ peaks,
                                                                double2* __restrict__ z) {
     __shared__ double2 x[kConvValues];
     __shared__ double2 tw[1 << (kConvMaxLog / 2)];
     const ConvTerm t = blockIdx.y ? t1 : t0;
     const int lc = kConvMinLog - lg1, C = 1 << lc;  // kConvValues = 2^kConvMinLog
     const uint32_t c0 = blockIdx.x << lc;
+    const Level la = level_of(peaks, 2 * blockIdx.y), lb = level_of(peaks, 2 * blockIdx.y + 1);
+    if (nothing(la, lb)) return;  // k_conv_rows leaves the term out
+    const double sa = ldexp(1.0, -la.exponent()), sb = ldexp(1.0, -lb.exponent());
     fill_roots(tw, lg1);
     for (int e = (int)threadIdx.x; e < kConvValues; e += kConvThreads) {
         const uint32_t n1 = (uint32_t)e >> lc, c = (uint32_t)e & (C - 1), n = (n1 << lg2) + c0 + c;
-        x[(c << lg1) + n1] = make_double2(n < t.n_track ? (double)t.track[n] : 0.0,
-                                          n < t.n_signal ? (double)t.signal[n] : 0.0);
+        x[(c << lg1) + n1] = make_double2(n < t.n_track ? (double)t.track[n] * sa : 0.0,
+                                          n < t.n_signal ? (double)t.signal[n] * sb : 0.0);
     }
     __syncthreads();
     lds_fft<false>(x, tw, lg1, C);
@@ -167,7 +218,9 @@ __global__ void __launch_bounds__(kConvThreads) k_conv_columns(ConvTerm t0, Conv
 
 // block k1 = 0 .. N1 / 2: rows k1 and N1 - k1 of every term; the product's
 // rows replace the first term's
-__global__ void __launch_bounds__(kConvThreads) k_conv_rows(int terms, int lg1, int lg2, double2* __restrict__ z) {
+__global__ void __launch_bounds__(kConvThreads) k_conv_rows(int terms, int lg1, int lg2,
+                                                            const uint32_t* __restrict__ peaks,
+                                                            double2* __restrict__ z) {
     __shared__ double2 x[kConvValues];
     __shared__ double2 tw[1 << (kConvMaxLog / 2)];
     constexpr int kPer = kConvValues / 2 / kConvThreads;  // frequencies per thread and row
@@ -180,6 +233,9 @@ __global__ void __launch_bounds__(kConvThreads) k_conv_rows(int terms, int lg1, 
     // frequency -k of [ra][k2] is [rb][mirror(k2)]
     auto mirror = [&](int k2) { return ra == 0 ? (N2 - k2) & (N2 - 1) : N2 - 1 - k2; };
     for (int t = 0; t < terms; ++t) {
+        const Level la = level_of(peaks, 2 * t), lb = level_of(peaks, 2 * t + 1);
+        if (nothing(la, lb)) continue;
+        const double back = ldexp(1.0, la.exponent() + lb.exponent());
         const double2* in = z + ((size_t)t << (lg1 + lg2));
         for (int e = (int)threadIdx.x; e < 2 * N2; e += kConvThreads)
             x[e] = in[((size_t)(e < N2 ? ra : rb) << lg2) + (e & (N2 - 1))];
@@ -194,8 +250,8 @@ __global__ void __launch_bounds__(kConvThreads) k_conv_rows(int terms, int lg1, 
                 const double2 A = make_double2(0.5 * (u.x + v.x), 0.5 * (u.y - v.y));
                 const double2 B = make_double2(0.5 * (u.y + v.y), 0.5 * (v.x - u.x));
                 const double2 P = cmul(A, B);
-                acc[j].x += P.x;
-                acc[j].y += P.y;
+                acc[j].x += P.x * back;
+                acc[j].y += P.y * back;
             }
         }
         __syncthreads();
@@ -240,12 +296,13 @@ ear_status convolve_short(Ctx* c, const float* const* tracks, const uint32_t* n_
                           uint32_t terms, uint32_t n_sig, float* out, uint32_t n_out, int lg) {
     const int lg2 = lg / 2, lg1 = lg - lg2;
     hipStream_t st = c->stream;
-    DevBuf in(c), z(c), res(c);
+    DevBuf in(c), z(c), res(c), peaks(c);
     size_t n_in = (size_t)terms * n_sig;
     for (uint32_t t = 0; t < terms; ++t) n_in += n_track[t];
     TRY(in.alloc(n_in * sizeof(float)));
     TRY(z.alloc(((size_t)terms << lg) * sizeof(double2)));
     TRY(res.alloc((size_t)n_out * sizeof(float)));
+    TRY(peaks.alloc(2 * terms * kPeakBlocks * sizeof(uint32_t)));
     ConvTerm term[2] = {};
     float* p = in.as<float>();
     for (uint32_t t = 0; t < terms; ++t) {
@@ -255,8 +312,11 @@ ear_status convolve_short(Ctx* c, const float* const* tracks, const uint32_t* n_
         p += n_track[t] + n_sig;
     }
     const uint32_t cols = (1u << lg2) >> (kConvMinLog - lg1);  // workgroups of columns
-    k_conv_columns<<<dim3(cols, terms), kConvThreads, 0, st>>>(term[0], term[1], lg1, lg2, z.as<double2>());
-    k_conv_rows<<<(1u << lg1) / 2 + 1, kConvThreads, 0, st>>>((int)terms, lg1, lg2, z.as<double2>());
+    k_conv_peaks<<<dim3(kPeakBlocks, 2 * terms), kConvThreads, 0, st>>>(term[0], term[1], peaks.as<uint32_t>());
+    k_conv_columns<<<dim3(cols, terms), kConvThreads, 0, st>>>(term[0], term[1], lg1, lg2, peaks.as<uint32_t>(),
+                                                               z.as<double2>());
+    k_conv_rows<<<(1u << lg1) / 2 + 1, kConvThreads, 0, st>>>((int)terms, lg1, lg2, peaks.as<uint32_t>(),
+                                                              z.as<double2>());
     k_conv_out<<<cols, kConvThreads, 0, st>>>(lg1, lg2, z.as<double2>(), n_out, res.as<float>());
     EAR_HIP_TRY(c, hipGetLastError());
     EAR_HIP_TRY(c, hipMemcpyAsync(out, res.p, (size_t)n_out * 4, hipMemcpyDeviceToHost, st));
