@@ -43,7 +43,6 @@ constexpr int kShadeBlock = 256;  // k_shade: its block-wide appends take one co
 constexpr uint32_t kNoallocWaves = 16;
 constexpr size_t kNoallocMinRays = 4096;
 constexpr double kBinMetres = 343.0 / 44100.0;       // a histogram bin as a distance
-constexpr uint64_t kRawStage = 64ull * 1024 * 1024;  // bytes of raw sums staged at a time
 
 enum StatIdx {
     ST_SEGMENTS = 0,
@@ -2140,10 +2139,11 @@ __global__ void __launch_bounds__(256) k_values(const InstDev* __restrict__ inst
 // own distance (33 bins at 3 s), so bins are independent: a grid over all of
 // them, where the prefix sums of k_finalize are one block per row (the hall's
 // 3 s stereo rows: 1.05 ms with 12 blocks, 0.1 ms here).  The rows must not be
-// written meanwhile: raw sums go to `raw` ([row][kind][bin], or null), rows
-// [row0, row0 + gridDim.y) of the table.
+// written meanwhile: raw sums go to `raw` ([row][kind][bin - bin0], or null),
+// bins [bin0, bin1) of rows [row0, row0 + gridDim.y) of the table.
 __global__ void __launch_bounds__(256) k_finish(const InstDev* __restrict__ inst, const uint4* __restrict__ rows,
-                                                uint32_t row0, unsigned long long* __restrict__ raw,
+                                                uint32_t row0, uint32_t bin0, uint32_t bin1,
+                                                unsigned long long* __restrict__ raw,
                                                 const uint64_t* __restrict__ raw_off) {
     const uint32_t row = row0 + blockIdx.y;
     const uint4 rw = rows[row];
@@ -2151,8 +2151,8 @@ __global__ void __launch_bounds__(256) k_finish(const InstDev* __restrict__ inst
     const RenderParams& P = In.P;
     const int band = (int)rw.y;
     const uint32_t ch = rw.z, nb = P.n_bins, n_ch = P.n_channels, kinds = P.hist_kinds;
-    const uint32_t j = blockIdx.x * 256 + threadIdx.x;
-    if (j >= nb) return;
+    const uint32_t j = bin0 + blockIdx.x * 256 + threadIdx.x, end = min(bin1, nb);
+    if (j >= end) return;
     const size_t r0 = (((size_t)band * n_ch + ch) * kinds) * nb;
     const ulonglong2* c0 = (const ulonglong2*)(In.hist + 4 * r0);  // [kind][parity][bin]
     // the two widths of ramps that start at s are wl and wl + 1: the least
@@ -2186,7 +2186,7 @@ __global__ void __launch_bounds__(256) k_finish(const InstDev* __restrict__ inst
     }
     if (raw)
         for (uint32_t k = 0; k < kinds; ++k) {
-            ulonglong2* o = (ulonglong2*)raw + raw_off[row] - raw_off[row0] + (size_t)k * nb + j;
+            ulonglong2* o = (ulonglong2*)raw + raw_off[row] - raw_off[row0] + (size_t)k * (end - bin0) + (j - bin0);
             *o = make_ulonglong2(v[k].lo, (unsigned long long)v[k].hi);
         }
     finished_values(In, band, ch, j, v);
@@ -2576,8 +2576,8 @@ ear_status run_batch(Ctx* c, uint32_t n_items, DeviceScene* const* scenes, const
             I.P.src_n_tris = m;
             I.P.src_total_area = total;
         }
-        // raw sums of one-point rows are staged beside them: the no-allocation
-        // render's region has no room set aside for that
+        // raw sums of one-point rows are staged in the overflow stacks, which the
+        // no-allocation render keeps small
         const bool raw1 = outs[i] && (outs[i]->raw || outs[i]->abs_raw);
         if (noalloc && raw1) I.P.one_point = 0;
         want_raw1 = want_raw1 || (raw1 && I.P.one_point);
@@ -3079,48 +3079,54 @@ ear_status run_batch(Ctx* c, uint32_t n_items, DeviceScene* const* scenes, const
         k_values<<<dim3((max_nb + 255) / 256, (uint32_t)vrows.size()), 256, 0, st>>>(di, dvrows.as<uint4>());
     }
     // One-point rows: finished in one launch, or where raw sums are wanted in
-    // runs of rows whose sums fit a staging buffer (at most kRawStage, in the
-    // memory that the ray queues, now done with, gave back).
+    // runs of rows (of bins, if a row is longer) whose sums fit the overflow
+    // stacks, which no walk uses any more.  (A buffer of their own made a render
+    // of few rays with long rows need more memory than its tracing.)
     if (!orows.empty()) {
         EAR_HIP_TRY(c, hipMemcpyAsync(dorows.p, orows.data(), sizeof(uint4) * orows.size(), hipMemcpyHostToDevice, st));
         EAR_HIP_TRY(c, hipMemcpyAsync(dorawo.p, raw_off.data(), 8 * raw_off.size(), hipMemcpyHostToDevice, st));
         const uint32_t n_or = (uint32_t)orows.size();
-        auto finish = [&](uint32_t r0, uint32_t n, unsigned long long* raw) {
+        auto finish = [&](uint32_t r0, uint32_t n, uint32_t b0, uint32_t b1, unsigned long long* raw) {
             for (uint32_t k = 0; k < n; k += 32768u)  // a grid's second dimension
-                k_finish<<<dim3((max_nb1 + 255) / 256, std::min(n - k, 32768u)), 256, 0, st>>>(
-                    di, dorows.as<uint4>(), r0 + k, raw ? raw + 2 * (raw_off[r0 + k] - raw_off[r0]) : nullptr,
+                k_finish<<<dim3((b1 - b0 + 255) / 256, std::min(n - k, 32768u)), 256, 0, st>>>(
+                    di, dorows.as<uint4>(), r0 + k, b0, b1, raw ? raw + 2 * (raw_off[r0 + k] - raw_off[r0]) : nullptr,
                     dorawo.as<uint64_t>());
         };
-        if (!want_raw1) {
-            finish(0, n_or, nullptr);
-        } else {
-            EAR_HIP_TRY(c, hipStreamSynchronize(st));
-            for (DevBuf* b : {&qo[0], &qo[1], &qd[0], &qd[1], &qm[0], &qm[1], &hits, &so, &sm}) b->release();
-            uint64_t most = 0;
-            for (uint32_t r = 0; r < n_or; ++r) most = std::max(most, raw_off[r + 1] - raw_off[r]);
-            DevBuf stage(c);
-            const uint64_t cells = std::max(most, std::min<uint64_t>(raw_off[n_or], kRawStage / 16));
-            TRY(stage.alloc(cells * 16));
-            for (uint32_t r0 = 0; r0 < n_or;) {
-                uint32_t r1 = r0 + 1;
-                while (r1 < n_or && raw_off[r1 + 1] - raw_off[r0] <= cells) ++r1;
-                finish(r0, r1 - r0, stage.as<unsigned long long>());
-                EAR_HIP_TRY(c, hipGetLastError());
-                for (uint32_t r = r0; r < r1; ++r) {
-                    const uint4 w = orows[r];
-                    const RenderParams& P = inst[w.x].P;
-                    for (uint32_t k = 0; outs[w.x] && k < P.hist_kinds; ++k) {
-                        int64_t* raw = k == 0 ? outs[w.x]->raw : outs[w.x]->abs_raw;
-                        if (raw)
-                            EAR_HIP_TRY(c, hipMemcpyAsync(raw + 2 * ((size_t)w.y * P.n_channels + w.z) * P.n_bins,
-                                                          stage.as<unsigned long long>() +
-                                                              2 * (raw_off[r] - raw_off[r0] + (uint64_t)k * P.n_bins),
-                                                          (size_t)P.n_bins * 16, hipMemcpyDeviceToHost, st));
-                    }
-                }
-                EAR_HIP_TRY(c, hipStreamSynchronize(st));
-                r0 = r1;
+        unsigned long long* stage = gs.as<unsigned long long>();
+        const uint64_t cells = gs.n / 16;
+        // bins [b0, b1) of row r, staged from cell `from` on, to the caller
+        auto copy_raw = [&](uint32_t r, uint32_t b0, uint32_t b1, uint64_t from) -> ear_status {
+            const uint4 w = orows[r];
+            const RenderParams& P = inst[w.x].P;
+            for (uint32_t k = 0; outs[w.x] && k < P.hist_kinds; ++k) {
+                int64_t* raw = k == 0 ? outs[w.x]->raw : outs[w.x]->abs_raw;
+                if (raw)
+                    EAR_HIP_TRY(c, hipMemcpyAsync(raw + 2 * (((size_t)w.y * P.n_channels + w.z) * P.n_bins + b0),
+                                                  stage + 2 * (from + (uint64_t)k * (b1 - b0)), (size_t)(b1 - b0) * 16,
+                                                  hipMemcpyDeviceToHost, st));
             }
+            return EAR_OK;
+        };
+        if (!want_raw1) finish(0, n_or, 0, max_nb1, nullptr);
+        for (uint32_t r0 = 0; want_raw1 && r0 < n_or;) {
+            const RenderParams& P = inst[orows[r0].x].P;
+            uint32_t r1 = r0 + 1;
+            if (raw_off[r1] - raw_off[r0] > cells) {
+                const uint32_t per = (uint32_t)(cells / P.hist_kinds);
+                for (uint32_t b0 = 0; b0 < P.n_bins;) {
+                    const uint32_t b1 = P.n_bins - b0 > per ? b0 + per : P.n_bins;
+                    finish(r0, 1, b0, b1, stage);
+                    EAR_HIP_TRY(c, hipGetLastError());
+                    TRY(copy_raw(r0, b0, b1, 0));
+                    b0 = b1;
+                }
+            } else {
+                while (r1 < n_or && raw_off[r1 + 1] - raw_off[r0] <= cells) ++r1;
+                finish(r0, r1 - r0, 0, max_nb1, stage);
+                EAR_HIP_TRY(c, hipGetLastError());
+                for (uint32_t r = r0; r < r1; ++r) TRY(copy_raw(r, 0, inst[orows[r].x].P.n_bins, raw_off[r] - raw_off[r0]));
+            }
+            r0 = r1;
         }
     }
     EAR_HIP_TRY(c, hipGetLastError());
