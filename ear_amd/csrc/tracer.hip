@@ -3078,60 +3078,63 @@ ear_status run_batch(Ctx* c, uint32_t n_items, DeviceScene* const* scenes, const
         EAR_HIP_TRY(c, hipMemcpyAsync(dvrows.p, vrows.data(), sizeof(uint4) * vrows.size(), hipMemcpyHostToDevice, st));
         k_values<<<dim3((max_nb + 255) / 256, (uint32_t)vrows.size()), 256, 0, st>>>(di, dvrows.as<uint4>());
     }
-    // One-point rows: finished in one launch, or where raw sums are wanted in
-    // runs of rows (of bins, if a row is longer) whose sums fit the overflow
-    // stacks, which no walk uses any more.  (A buffer of their own made a render
-    // of few rays with long rows need more memory than its tracing.)
-    if (!orows.empty()) {
+    // One-point rows: finished in one launch.  Raw sums that are wanted go to the
+    // overflow stacks, which no walk uses any more, and from there to the caller:
+    // all of them in that launch, or if they do not fit in runs of rows (of bins,
+    // if a row is longer) finished again after the render's time is taken.  (A
+    // buffer of their own made a render of few rays with long rows need more
+    // memory than its tracing.)
+    const uint32_t n_or = (uint32_t)orows.size();
+    unsigned long long* stage = gs.as<unsigned long long>();
+    const uint64_t cells = gs.n / 16;
+    const bool whole = raw_off[n_or] <= cells;
+    auto finish = [&](uint32_t r0, uint32_t n, uint32_t b0, uint32_t b1, unsigned long long* raw) {
+        for (uint32_t k = 0; k < n; k += 32768u)  // a grid's second dimension
+            k_finish<<<dim3((b1 - b0 + 255) / 256, std::min(n - k, 32768u)), 256, 0, st>>>(
+                di, dorows.as<uint4>(), r0 + k, b0, b1, raw ? raw + 2 * (raw_off[r0 + k] - raw_off[r0]) : nullptr,
+                dorawo.as<uint64_t>());
+    };
+    if (n_or) {
         EAR_HIP_TRY(c, hipMemcpyAsync(dorows.p, orows.data(), sizeof(uint4) * orows.size(), hipMemcpyHostToDevice, st));
         EAR_HIP_TRY(c, hipMemcpyAsync(dorawo.p, raw_off.data(), 8 * raw_off.size(), hipMemcpyHostToDevice, st));
-        const uint32_t n_or = (uint32_t)orows.size();
-        auto finish = [&](uint32_t r0, uint32_t n, uint32_t b0, uint32_t b1, unsigned long long* raw) {
-            for (uint32_t k = 0; k < n; k += 32768u)  // a grid's second dimension
-                k_finish<<<dim3((b1 - b0 + 255) / 256, std::min(n - k, 32768u)), 256, 0, st>>>(
-                    di, dorows.as<uint4>(), r0 + k, b0, b1, raw ? raw + 2 * (raw_off[r0 + k] - raw_off[r0]) : nullptr,
-                    dorawo.as<uint64_t>());
-        };
-        unsigned long long* stage = gs.as<unsigned long long>();
-        const uint64_t cells = gs.n / 16;
-        // bins [b0, b1) of row r, staged from cell `from` on, to the caller
-        auto copy_raw = [&](uint32_t r, uint32_t b0, uint32_t b1, uint64_t from) -> ear_status {
-            const uint4 w = orows[r];
-            const RenderParams& P = inst[w.x].P;
-            for (uint32_t k = 0; outs[w.x] && k < P.hist_kinds; ++k) {
-                int64_t* raw = k == 0 ? outs[w.x]->raw : outs[w.x]->abs_raw;
-                if (raw)
-                    EAR_HIP_TRY(c, hipMemcpyAsync(raw + 2 * (((size_t)w.y * P.n_channels + w.z) * P.n_bins + b0),
-                                                  stage + 2 * (from + (uint64_t)k * (b1 - b0)), (size_t)(b1 - b0) * 16,
-                                                  hipMemcpyDeviceToHost, st));
-            }
-            return EAR_OK;
-        };
-        if (!want_raw1) finish(0, n_or, 0, max_nb1, nullptr);
-        for (uint32_t r0 = 0; want_raw1 && r0 < n_or;) {
-            const RenderParams& P = inst[orows[r0].x].P;
-            uint32_t r1 = r0 + 1;
-            if (raw_off[r1] - raw_off[r0] > cells) {
-                const uint32_t per = (uint32_t)(cells / P.hist_kinds);
-                for (uint32_t b0 = 0; b0 < P.n_bins;) {
-                    const uint32_t b1 = P.n_bins - b0 > per ? b0 + per : P.n_bins;
-                    finish(r0, 1, b0, b1, stage);
-                    EAR_HIP_TRY(c, hipGetLastError());
-                    TRY(copy_raw(r0, b0, b1, 0));
-                    b0 = b1;
-                }
-            } else {
-                while (r1 < n_or && raw_off[r1 + 1] - raw_off[r0] <= cells) ++r1;
-                finish(r0, r1 - r0, 0, max_nb1, stage);
-                EAR_HIP_TRY(c, hipGetLastError());
-                for (uint32_t r = r0; r < r1; ++r) TRY(copy_raw(r, 0, inst[orows[r].x].P.n_bins, raw_off[r] - raw_off[r0]));
-            }
-            r0 = r1;
-        }
+        finish(0, n_or, 0, max_nb1, want_raw1 && whole ? stage : nullptr);
     }
     EAR_HIP_TRY(c, hipGetLastError());
     if (t1) EAR_HIP_TRY(c, hipEventRecord(t1, st));
     EAR_HIP_TRY(c, hipStreamSynchronize(st));
+    // bins [b0, b1) of row r, staged from cell `from` on, to the caller
+    auto copy_raw = [&](uint32_t r, uint32_t b0, uint32_t b1, uint64_t from) -> ear_status {
+        const uint4 w = orows[r];
+        const RenderParams& P = inst[w.x].P;
+        for (uint32_t k = 0; outs[w.x] && k < P.hist_kinds; ++k) {
+            int64_t* raw = k == 0 ? outs[w.x]->raw : outs[w.x]->abs_raw;
+            if (raw)
+                EAR_HIP_TRY(c, hipMemcpyAsync(raw + 2 * (((size_t)w.y * P.n_channels + w.z) * P.n_bins + b0),
+                                              stage + 2 * (from + (uint64_t)k * (b1 - b0)), (size_t)(b1 - b0) * 16,
+                                              hipMemcpyDeviceToHost, st));
+        }
+        return EAR_OK;
+    };
+    for (uint32_t r0 = 0; want_raw1 && r0 < n_or;) {
+        const RenderParams& P = inst[orows[r0].x].P;
+        uint32_t r1 = r0 + 1;
+        if (raw_off[r1] - raw_off[r0] > cells) {
+            const uint32_t per = (uint32_t)(cells / P.hist_kinds);
+            for (uint32_t b0 = 0; b0 < P.n_bins;) {
+                const uint32_t b1 = P.n_bins - b0 > per ? b0 + per : P.n_bins;
+                finish(r0, 1, b0, b1, stage);
+                EAR_HIP_TRY(c, hipGetLastError());
+                TRY(copy_raw(r0, b0, b1, 0));
+                b0 = b1;
+            }
+        } else {
+            while (r1 < n_or && raw_off[r1 + 1] - raw_off[r0] <= cells) ++r1;
+            if (!whole) finish(r0, r1 - r0, 0, max_nb1, stage);
+            EAR_HIP_TRY(c, hipGetLastError());
+            for (uint32_t r = r0; r < r1; ++r) TRY(copy_raw(r, 0, inst[orows[r].x].P.n_bins, raw_off[r] - raw_off[r0]));
+        }
+        r0 = r1;
+    }
 
     // copy out [band slot][channel][bin] rows of every rendered band
     for (uint32_t i = 0; i < n_items; ++i) {

@@ -1,5 +1,6 @@
 """Raw sums returned to the caller: no more device memory than the same render
-without them, however few rays and long rows, and in whatever pieces."""
+without them, however few rays and long rows, in whatever pieces, and outside
+the render's device time."""
 import numpy as np
 import pytest
 
@@ -58,3 +59,18 @@ def test_rows_longer_than_the_staging_memory(gpu_ctx, abs_hist):
     if abs_hist:
         np.testing.assert_array_equal(few.abs_raw, ref.abs_raw)
         np.testing.assert_array_equal(few.abs_value, ref.abs_value)
+
+
+@pytest.mark.parametrize("waves_per_cu", [0, 1])
+def test_device_time_leaves_the_copies_of_raw_sums_out(gpu_ctx, waves_per_cu):
+    """trace_ms is the device time of the render: the copies of 100 MB of raw
+    sums (10 ms at 10 GB/s) are no part of it."""
+    s = scenes.shoebox()
+    gpu_ctx.set_tuning(waves_per_cu=waves_per_cu)
+    try:
+        with api.Scene(gpu_ctx, s["tris"], s["mat"], s["materials"]) as sc:
+            ms = {raw: min(api.render(gpu_ctx, sc, **_kw(s, n_bins=2 * BINS, want_raw=raw)).stats["trace_ms"]
+                           for _ in range(5)) for raw in (False, True)}
+    finally:
+        gpu_ctx.set_tuning()
+    assert ms[True] < 1.5 * ms[False] + 1.0
