@@ -561,7 +561,11 @@ struct Walker<LDS, BLOCK, 4, ANY, INSTR> {
         best_t = t_max;
         best_s = -1;
         best_o = 0;
-        cur = T.n_tris != 0 ? 0 : kIdle;
+        // an origin that is no number on any axis is in no box (the minima and
+        // maxima of visit() pass over a NaN, so it would be in all of them)
+        const float px = o.x * ix, py = o.y * iy, pz = o.z * iz;
+        const bool nowhere = (px != px) & (py != py) & (pz != pz);
+        cur = T.n_tris != 0 && !nowhere ? 0 : kIdle;
         stk.sp = 0;
     }
 
