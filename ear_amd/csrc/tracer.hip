@@ -303,7 +303,10 @@ struct Claim {
         next = end = fails = 0;
         // entries per atomic: what one refill needs, or while the queue is
         // long (256 for every wave) enough for several refills
-        want = f.chunk ? f.chunk : (n / 256u >= threads / 64u ? 64u : 0u);
+        // (a chunk so large that the waves' last, failing claims wrap a counter
+        // would hand its segment out again: at most n + chunk (waves + n_seg))
+        want = f.chunk ? min(f.chunk, (0xFFFFFFFFu - n) / (threads / 64u + n_seg))
+                       : (n / 256u >= threads / 64u ? 64u : 0u);
         if (n <= threads) {
             const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)((threadIdx.x >> 6) * gridDim.x + blockIdx.x));
             next = min(wave * own, n);
