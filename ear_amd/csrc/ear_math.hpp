@@ -290,7 +290,6 @@ EAR_HD V3 blend_spec(V3 v, V3 refl, float f) {
     V3 w{v.x * g + refl.x * f, v.y * g + refl.y * f, v.z * g + refl.z * f};
     return normalized(w);
 }
-EAR_HD V3 sample_hemi_spec(Rng& r, V3 n, V3 refl, float f) { return blend_spec(sample_hemi(r, n), refl, f); }
 
 // ---------------------------------------------------------------------------
 // The score form of the specularity gradient.  v = normalize((1-s) h + s r),
