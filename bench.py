@@ -16,15 +16,18 @@ over its HIP-event time (kernel_rooflines below), with node visits V and
 triangle tests T per query counted by an instrumented pass over the same rays;
 `roofline` is the dominant one (the largest time per render), and
 `render_roofline` the whole render at bytes per segment.  `traffic` is
-rocprofv3's FETCH_SIZE + WRITE_SIZE per launch where profiles/ holds it.
+rocprofv3's FETCH_SIZE + WRITE_SIZE per launch where profiles/ holds it for the
+kernels as they are built now, else null (measured_traffic below).
 `cpu_baseline` is the CPU oracle (a brute-force restatement of the reference
 algorithm) timed on this host on the first K rays of the same Philox streams.
 """
 from __future__ import annotations
 
 import argparse
+import hashlib
 import json
 import os
+import re
 import sys
 import time
 
@@ -249,6 +252,30 @@ def main():
     print(json.dumps(out), flush=True)
 
 
+def kernel_source_id():
+    """Of the tracing kernels' source without its comments and white space: two
+    builds of the same id move the same bytes."""
+    h = hashlib.sha256()
+    for name in ("ear_internal.hpp", "ear_math.hpp", "lbvh.hip", "tracer.hip"):
+        with open(os.path.join(ROOT, "ear_amd", "csrc", name)) as f:
+            h.update(re.sub(r"\s+", "", re.sub(r"//.*", "", f.read())).encode())
+    return h.hexdigest()[:16]
+
+
+def measured_traffic(path, units_per_launch):
+    """Bytes per launch measured for this build of a kernel, on launches of this
+    many units of work (within 2%); None where the file is of others."""
+    if not os.path.exists(path):
+        return None
+    with open(path) as f:
+        t = json.load(f)
+    if t.get("kernel_source") != kernel_source_id():
+        return None
+    if abs(units_per_launch / max(1e-9, t.get("units_per_launch", 0.0)) - 1.0) > 0.02:
+        return None
+    return t["bytes_per_launch"]
+
+
 def kernel_rooflines(acc, ist, info, traffic_dir, steps):
     """Algorithmic-byte rooflines of the bounce loop's kernels over the timed
     renders (acc: summed ear_stats), with node visits V and triangle tests T
@@ -261,10 +288,12 @@ def kernel_rooflines(acc, ist, info, traffic_dir, steps):
       k_shadow_f per shadow query: 32 (request) + B V_sh + 36 T_sh, plus per
         ramp 16 (its 128-bit point) with direct atomics, or with the
         time-tiled splat 4 per record slot + 8 per record
-    B = 64 bytes per node visit.  `traffic` is rocprofv3's FETCH_SIZE +
-    WRITE_SIZE per launch of that kernel (scaled by a plain copy), where
-    profiles/ holds it for the kernel; measured_frac = traffic per average
-    launch time over the peak."""
+    B = 64 bytes per node visit.  These bytes are mostly served by the caches,
+    so a fraction above 1 says that HBM is not the bound.  `traffic` is
+    rocprofv3's FETCH_SIZE + WRITE_SIZE per launch of that kernel (scaled by a
+    plain copy), where profiles/ holds it for this kernel and this length of its
+    launches (measured_traffic); measured_frac = traffic per average launch time
+    over the peak."""
     B = info["node_bytes"]
     qe, qs = max(1, acc["extend_queries"]), max(1, acc["shadow_queries"])
     V = ist["node_visits_closest"] / max(1, ist["extend_queries"])
@@ -286,11 +315,7 @@ def kernel_rooflines(acc, ist, info, traffic_dir, steps):
     for k, (bpu, units, ms, launches, unit) in per.items():
         achieved = bpu * units / max(1e-9, ms * 1e-3) / 1e9
         avg_ms = ms / max(1, launches)
-        traffic = None
-        tf = os.path.join(traffic_dir, f"traffic_{k}_hall200k.json")
-        if os.path.exists(tf):
-            with open(tf) as f:
-                traffic = json.load(f).get("bytes_per_launch")
+        traffic = measured_traffic(os.path.join(traffic_dir, f"traffic_{k}_hall200k.json"), units / max(1, launches))
         out[k] = {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                   "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": traffic,
                   "measured_frac": (round(traffic / (avg_ms * 1e-3) / 1e9 / HBM_PEAK_GBS, 4) if traffic else None),
