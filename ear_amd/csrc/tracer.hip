@@ -533,9 +533,13 @@ struct Walker {
 // one (whichever more of the wave's walks are at), so that no step runs both
 // for a few lanes each.  Hall of 200k triangles, 3 x 10M rays: closest hit
 // 176 -> 128 ms and any hit 137 -> 92 ms per render (1.34e11 -> 7.8e10 vector
-// instructions); each lane's 16-byte piece of a node or triangle is an L1
-// access of its own, 72 per closest-hit query, and the L1 takes one per clock
-// and CU: that is now the closest-hit kernel's bound (1.0 measured).
+// instructions).  A lane's 16-byte piece of a node or triangle is an L1 access
+// of its own unless another lane reads the same, 63 per closest-hit query, and
+// the L1 takes one per clock and CU: that is now the closest-hit kernel's bound
+// (1.02 measured).  Popped children are not held against the best hit, and an
+// any-hit walk takes children unsorted: 5.66 triangle tests a closest-hit query
+// where the walk that held leaves back made 5.31, 9.54 node visits a shadow
+// query for 8.90 (2.85 triangle tests for 3.13).
 template <int LDS, int BLOCK, bool ANY, bool INSTR>
 struct Walker<LDS, BLOCK, 4, ANY, INSTR> {
     static constexpr int kIdle = kEmpty4;  // above every node index
@@ -816,7 +820,7 @@ __device__ uint32_t splat_ramp(unsigned long long* h, uint32_t nb, uint32_t one,
 // time tile of kTile bins).  Per bounce iteration a counting sort groups the
 // records by key (k_tile_count, k_tile_scan, k_tile_scatter), and
 // k_tile_splat cuts the sorted records into chunks of kTileChunk, one
-// workgroup each: for every key among its records it adds the three points of
+// workgroup each: for every key among its records it adds the points of
 // each ramp into a 128-bit accumulator tile in LDS (64-bit LDS atomics with an
 // explicit carry), then adds that tile to the row in HBM, one global 128-bit
 // add per touched bin.  The rays of one bounce iteration have travelled
@@ -1306,7 +1310,9 @@ __global__ void __launch_bounds__(kShadeBlock, 6) k_shade(const InstDev* __restr
         // NEE to every recorder (src/Scene.cpp:185-268).  The slots of the
         // connections and of the continuing rays come from one append, so the
         // connections are counted before they are stored; the first two
-        // recorders' weights are kept for that, the others' computed again.
+        // recorders' weights are kept for that, the others' computed again
+        // (the 200k hall of 3 x 3M rays with 8 recorders: 290 ms, 548 with an
+        // append and one weight per recorder).
         auto weight = [&](uint32_t r, float& c) -> bool {
             if (!(alive && nee && r < n_rec)) return false;
             const RenderParams& P = inst[id].P;
@@ -2994,7 +3000,11 @@ ear_status run_batch(Ctx* c, uint32_t n_items, DeviceScene* const* scenes, const
     // 32 rooms at 2^20, 2^21, 2^22, all: 116, 113, 110, 100 ms; the 200k hall
     // 326, 321, 319, 356; 12 keyframes of the 100k hall 72.3, 72.2, 74.0,
     // 86.7: rooms would take more, halls do not, and their trees do not tell
-    // them apart; 1: no tail launch)
+    // them apart; 1: no tail launch.  Renders wholly below it, from the first
+    // segment in the tail against the last 2^20 and against no tail: the 200k
+    // hall of 3 x 200k rays 14.9, 15.0, 31.5 ms, of 3 x 500k 27.6, 30.3, 41.6,
+    // of 3 x 650k 32.6, 34.6, 46.2; a 20k hall 24.3, 27.7, 35.0 and a 500k hall
+    // 45.9, 46.0, 63.1 of 3 x 650k; a 50k room 24.0, 36.8, 42.3)
     uint32_t max_tris = 0;
     for (uint32_t i = 0; i < n_items; ++i) max_tris = std::max(max_tris, inst[i].n_tris);
     const uint32_t tail_default = max_tris <= 64 ? 0xFFFFFFFFu : (1u << 21);

@@ -352,9 +352,11 @@ ear_status ear_render_backward_batch(ear_ctx* ctx, const ear_backward_item* item
  * convolution of ir with the signal; when ir2 is given (the keyframe
  * cross-fade, src/Recorder.cpp:233-243) the signal is faded out linearly
  * over its length for ir and faded in for ir2, and the two are added.  The
- * fades follow the reference's running-sum factors.  Single precision
- * (float FFTs): results agree with an exact convolution to about 1e-6 of the
- * largest output sample. */
+ * fades follow the reference's running-sum factors.  Up to n_out = 2^22 the
+ * transforms are in binary64, and the result is the exact convolution rounded
+ * to float (2^-24 of the largest output sample), whatever the sizes of the
+ * response and the signal; a silent response or signal gives zeros.  Longer
+ * ones use float FFTs and agree to about 1e-6 of the largest output sample. */
 ear_status ear_convolve(ear_ctx* ctx, const float* ir, uint32_t n_ir, const float* ir2, uint32_t n_ir2,
                         const float* signal, uint32_t n_sig, float* out);
 
