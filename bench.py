@@ -322,6 +322,9 @@ def kernel_rooflines(acc, ist, info, traffic_dir, steps):
                   "bytes_per_unit": round(bpu, 1), "unit_of_work": unit,
                   "units_per_launch": round(units / max(1, launches), 1), "avg_launch_ms": round(avg_ms, 4),
                   "launches": launches, "ms_per_render": round(ms / steps, 2)}
+    for k in ("k_extend_f", "k_shadow_f"):
+        out[k]["note"] = ("priced at HBM's peak, but the caches serve most of these bytes (traffic is what reaches "
+                          "HBM): the L1's access rate is what bounds the walk, profiles/pmc_l1_hall200k_10Mrays.txt")
     out["k_extend_f"].update(node_visits_per_query=round(V, 3), tri_tests_per_query=round(T, 3))
     out["k_shadow_f"].update(node_visits_per_query=round(Vs, 3), tri_tests_per_query=round(Ts, 3),
                              ramps_per_query=round(ramps_per_q, 4), splat="tiled" if tiled else "atomic")
